@@ -345,7 +345,6 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
     D.trisPerLane = sched.trisPerLane;
     D.batchShift = 0;   // log2(triangles per batch)
     while ((1u << D.batchShift) < D.block * D.trisPerLane) D.batchShift++;
-    const uint64_t batchTris = 1ull << D.batchShift;
     // pairs of consecutive triangles per lane (k_stage1_pairs), for draws
     // large enough that every wave of the grid claims many 128-triangle
     // batches (a small draw keeps the short per-batch walk of k_stage1).  An
@@ -361,6 +360,26 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
                                (D.block / 64);
         D.runs = tris >= 16ull * 128ull * waves;
     }
+
+    // few triangles per pixel: each covers several samples, and the draw is
+    // bound by its rasterisation (k_stage1_coarse).  The tuning's knobs of
+    // the other kernels (an explicit block, triangles per lane or walk) keep it off.
+    if (numViews == 1 && !manyInstances && !D.runs && tu.stage1_tris_per_lane == 0 && tu.stage1_layout != 0 &&
+        D.block == 256 && tu.stage1_fast_tiny == 0) {
+        uint64_t tris = 0;
+        for (uint32_t k = 0; k < D.numItems; k++)
+            tris += (uint64_t)list[k].numTriangles * (instanced ? (uint64_t)std::max(list[k].instances.count, 0) : 1u);
+        const uint64_t pixels = (uint64_t)targets[0].width * (uint64_t)targets[0].height;
+        D.coarse = tris <= kCoarseMaxTris && tris <= kCoarseTrisPerPixel * pixels;
+        if (D.coarse) {
+            // as many lanes per triangle as keep the draw's waves resident at once (32 per CU)
+            const uint64_t lanes = (uint64_t)ctx->numCUs * 32u * 64u;
+            while (D.splitShift < kCoarseMaxSplit && (tris << (D.splitShift + 1u)) <= lanes) D.splitShift++;
+            D.trisPerLane = 1;
+            D.batchShift = 8u - D.splitShift;
+        }
+    }
+    const uint64_t batchTris = 1ull << D.batchShift;
 
     D.items.resize(D.numItems);
     for (uint32_t k = 0; k < D.numItems; k++) {
@@ -442,7 +461,7 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
     D.offViews = align_up(D.offPrefix + (prefix ? D.inst.size() * sizeof(uint64_t) : 0), 256);
     D.offXf = align_up(D.offViews + (size_t)numViews * sizeof(ViewParams), 256);
     D.metaBytes = D.offXf + D.xf.size() * sizeof(Transform);
-    if (sched.wavesPerCU == 0) {
+    if (sched.wavesPerCU == 0 || D.coarse) {   // one workgroup per batch
         D.g1 = (uint32_t)std::min<uint64_t>(D.batches, 1ull << 31);
     } else {
         D.g1 = grid_for(ctx, sched.wavesPerCU, D.block / 64);
@@ -485,6 +504,7 @@ RasterParams plan_write(crx_context* ctx, const DrawPlan& D, char* host, char* d
     P.smallThreshold = tu.small_threshold;
     P.tile = (int32_t)tu.tile_size;
     P.batchShift = D.batchShift;
+    P.splitShift = D.splitShift;
     P.order = tu.stage1_order;
     // cull order 3 decides per item; a draw of several views tests backfaces
     // first (10.70 ms against 11.07 ms for frustum first on 64 views)
@@ -511,6 +531,8 @@ hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& D, const RasterParam
     record(ctx, T_S1, stream);
     if (D.numViews == 1 && !viewsKernel && D.runs)
         e = launch_stage1_pairs(P, D.block, D.g1, D.pu16, stream);
+    else if (D.numViews == 1 && !viewsKernel && D.coarse)
+        e = launch_stage1_coarse(P, D.g1, D.pu16, stream);
     else if (D.numViews == 1 && !viewsKernel)
         e = launch_stage1(P, D.block, D.trisPerLane, D.g1, D.pu16, D.instanceBoxes, stream);
     else e = launch_stage1_views(P, D.block, D.trisPerLane, D.g1, D.pu16, stream);

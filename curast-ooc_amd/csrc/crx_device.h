@@ -120,6 +120,17 @@ struct ViewParams {
 // boxes and tests them per instance (the reduction is paid once per batch).
 constexpr uint32_t kBoxInstances = 4;
 
+// A single-view draw of at most this many triangles, and triangles per pixel
+// of its target, takes k_stage1_coarse.  Stage 1 measured against k_stage1 on
+// spheres: 0.52 triangles per pixel (1 M at 1080p) 60 against 95 us, 2.0 26
+// against 38, 4.05 46 against 52, 8.1 82 against 88, 16 (8.4 M) 140 against
+// 129.  On terrains seen whole, which have less to rasterise, the loads that
+// k_stage1 prefetches weigh more with size: 1 M at 4K 36 against 51 us, 2 M
+// at 1080p 27 against 25, 3.9 M at 4K 54 against 50, 8 M at 4K 91 against 71.
+constexpr uint64_t kCoarseTrisPerPixel = 4;
+constexpr uint64_t kCoarseMaxTris = 3000000;
+constexpr uint32_t kCoarseMaxSplit = 4;   // most lanes (log2) that share a triangle
+
 constexpr uint32_t kViewShift = 24;                 // instance field: view << 24 | instance
 constexpr uint32_t kInstanceMask = (1u << 24) - 1u;
 constexpr uint32_t kMaxViews = 256;
@@ -148,7 +159,7 @@ struct RasterParams {
     uint32_t fastTiny;       // filtered tiny-triangle cull (crx_tuning::stage1_fast_tiny)
     uint32_t numWaves2;      // waves in the stage-2 grid
     uint32_t numWaves3;      // waves in the stage-3 grid
-    uint32_t pad0;
+    uint32_t splitShift;     // k_stage1_coarse: log2(lanes per triangle)
     uint32_t* claims;        // k_stage1_pairs: the per-XCD unit counters (CTR_CLAIM of the counter block)
 };
 

@@ -126,6 +126,8 @@ struct DrawPlan {
     uint32_t block = 256, trisPerLane = 1, batchShift = 8, g1 = 0, g2 = 0, g3 = 0;
     bool instanceBoxes = false;   // some item loops over >= 4 instances
     bool runs = false;            // k_stage1_runs (items carry the run layout; batches counts its units)
+    bool coarse = false;          // k_stage1_coarse (few triangles per pixel)
+    uint32_t splitShift = 0;      // its lanes per triangle (log2)
     bool prefix = false;          // the image carries the instances' triangle prefix (InstanceRec::cumm)
     size_t offItems = 0, offInst = 0, offPrefix = 0, offViews = 0, offXf = 0, metaBytes = 0;
 };

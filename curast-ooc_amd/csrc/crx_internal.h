@@ -26,6 +26,9 @@ hipError_t launch_store_view(const ViewParams& v, ViewParams* dst, hipStream_t s
 // let groups of triangles skip instances that cull them all as tiny)
 hipError_t launch_stage1(const RasterParams& P, uint32_t block, uint32_t trisPerLane, uint32_t grid, bool pu16,
                          bool instanceBoxes, hipStream_t stream);
+// Draws of few triangles per pixel, block 256: lane groups of 2^P.splitShift
+// per triangle (P.batchShift = 8 - P.splitShift), LDS raster tiles.
+hipError_t launch_stage1_coarse(const RasterParams& P, uint32_t grid, bool pu16, hipStream_t stream);
 // Pairs of consecutive triangles per lane, block 256 (k_stage1_pairs): the
 // items carry the strip layout (DrawItem::rowTris ...).
 hipError_t launch_stage1_pairs(const RasterParams& P, uint32_t block, uint32_t grid, bool pu16, hipStream_t stream);

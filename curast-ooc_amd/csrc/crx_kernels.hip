@@ -179,13 +179,27 @@ __device__ __forceinline__ VQ vertex_q(const float* m, f3 p) {
     return VQ{-xform_row(m, 2, p), xform_row(m, 1, p)};
 }
 
-template <bool PRE>
-__device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewParams& V, const float* __restrict__ m,
+//
+// DEFER: the function neither draws nor queues.  It tells what is to be done
+// with the triangle, for a caller that does it for its lanes together
+// (raster_wave), with the raster setup in *rt.
+enum S1Result : int { S1_NONE = 0, S1_RASTER = 1, S1_QUEUE = 2 };
+struct RasterTri {
+    float s, t;                          // at the box's first sample
+    float ds_dx, ds_dy, dt_dx, dt_dy;
+    float iza, izb, izc;
+    int32_t x, y, w, h;                  // box (w, h > 0)
+    bool fast;                           // depths in the range of the short reciprocal
+};
+
+template <bool PRE, bool DEFER = false>
+__device__ __forceinline__ S1Result stage1_core(const RasterParams& P, const ViewParams& V, const float* __restrict__ m,
                                             bool flip, f3 A, f3 B, f3 C, const VQ& qa, const VQ& qb, const VQ& qc,
-                                            uint64_t id, uint64_t queueEntry, uint32_t cullOrder) {
+                                            uint64_t id, uint64_t queueEntry, uint32_t cullOrder,
+                                            RasterTri* rt = nullptr) {
     const float da = qa.d, db = qb.d, dc = qc.d;
     // all vertices behind the camera (:119)
-    if (da <= 0.0f && db <= 0.0f && dc <= 0.0f) return;
+    if (da <= 0.0f && db <= 0.0f && dc <= 0.0f) return S1_NONE;
     bool nontrivial = (da <= 0.0f || db <= 0.0f || dc <= 0.0f);
     const bool safeDepth = (da >= 0x1p-102f && db >= 0x1p-102f && dc >= 0x1p-102f);
     const float fa = V.fa, f = V.f;
@@ -199,17 +213,17 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
         if (cullOrder == 1) {
             if (!PRE) { vya = xform_row(m, 1, A); vyb = xform_row(m, 1, B); vyc = xform_row(m, 1, C); }
             haveY = true;
-            if (frustum_culled_axis(f * vya, f * vyb, f * vyc, da, db, dc)) return;
+            if (frustum_culled_axis(f * vya, f * vyb, f * vyc, da, db, dc)) return S1_NONE;
             vxa = xform_row(m, 0, A); vxb = xform_row(m, 0, B); vxc = xform_row(m, 0, C);
             haveX = true;
-            if (frustum_culled_axis(fa * vxa, fa * vxb, fa * vxc, da, db, dc)) return;
+            if (frustum_culled_axis(fa * vxa, fa * vxb, fa * vxc, da, db, dc)) return S1_NONE;
         } else {
             vxa = xform_row(m, 0, A); vxb = xform_row(m, 0, B); vxc = xform_row(m, 0, C);
             haveX = true;
-            if (frustum_culled_axis(fa * vxa, fa * vxb, fa * vxc, da, db, dc)) return;
+            if (frustum_culled_axis(fa * vxa, fa * vxb, fa * vxc, da, db, dc)) return S1_NONE;
             if (!PRE) { vya = xform_row(m, 1, A); vyb = xform_row(m, 1, B); vyc = xform_row(m, 1, C); }
             haveY = true;
-            if (frustum_culled_axis(f * vya, f * vyb, f * vyc, da, db, dc)) return;
+            if (frustum_culled_axis(f * vya, f * vyb, f * vyc, da, db, dc)) return S1_NONE;
         }
     }
     if (!haveX) { vxa = xform_row(m, 0, A); vxb = xform_row(m, 0, B); vxc = xform_row(m, 0, C); }
@@ -224,12 +238,12 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
         const f3 ac = sub3(cv, av);
         float res = dot3(av, cross3(ab, ac));
         if (flip) res = -res;
-        if (res >= 0.0f) return;
+        if (res >= 0.0f) return S1_NONE;
     }
     if (!frustumFirst && !nontrivial) {
         if (safeDepth) {
             if (frustum_culled_axis(pxa, pxb, pxc, da, db, dc) || frustum_culled_axis(pya, pyb, pyc, da, db, dc))
-                return;
+                return S1_NONE;
         }
     }
     if (!nontrivial && !safeDepth) {
@@ -237,7 +251,7 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
         const float ay = pya / da, by = pyb / db, cy = pyc / dc;
         if ((ax > 1.0f && bx > 1.0f && cx > 1.0f) || (ax < -1.0f && bx < -1.0f && cx < -1.0f) ||
             (ay > 1.0f && by > 1.0f && cy > 1.0f) || (ay < -1.0f && by < -1.0f && cy < -1.0f))
-            return;
+            return S1_NONE;
     }
 
     // filtered tiny-triangle cull (see above); depths in [2^-100, 2^100]
@@ -255,7 +269,7 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
             const float hix = fminf(fmaxf(sxa, fmaxf(sxb, sxc)), V.Wm1);
             const float loy = fmaxf(fminf(sya, fminf(syb, syc)), 0.0f);
             const float hiy = fminf(fmaxf(sya, fmaxf(syb, syc)), V.Hm1);
-            if (surely_culled_axis(lox, hix, V.tinyMargin) || surely_culled_axis(loy, hiy, V.tinyMargin)) return;
+            if (surely_culled_axis(lox, hix, V.tinyMargin) || surely_culled_axis(loy, hiy, V.tinyMargin)) return S1_NONE;
         }
     }
 
@@ -270,7 +284,8 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
     const float dmin = fminf(da, fminf(db, dc)), dmax = fmaxf(da, fmaxf(db, dc));
     const float pmax = fmaxf(fmaxf(fmaxf(fabsf(pxa), fabsf(pxb)), fmaxf(fabsf(pxc), fabsf(pya))),
                              fmaxf(fabsf(pyb), fabsf(pyc)));
-    const bool fast = __ballot(!(dmin >= kDivLo && dmax <= kDivHi && pmax <= kDivHi)) == 0ull;
+    const bool inRange = dmin >= kDivLo && dmax <= kDivHi && pmax <= kDivHi;
+    const bool fast = __ballot(!inRange) == 0ull;
     float ax, bx, cx, ay, by, cy, iza, izb, izc;
     if (fast) {
         iza = rcp_refined(da);
@@ -307,8 +322,8 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
     if (!nontrivial) {
         const float sx = floorf(min_x);
         const float sy = floorf(min_y);
-        if (min_x > sx + 0.0f && max_x < sx + 1.0f + 0.0f) return;
-        if (min_y > sy + 0.0f && max_y < sy + 1.0f + 0.0f) return;
+        if (min_x > sx + 0.0f && max_x < sx + 1.0f + 0.0f) return S1_NONE;
+        if (min_y > sy + 0.0f && max_y < sy + 1.0f + 0.0f) return S1_NONE;
     }
 
     const int size_x = f2i(ceilf(max_x) - ceilf(min_x));
@@ -317,9 +332,10 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
     if (numFragments > P.smallThreshold) nontrivial = true;   // unsigned compare, as the reference
 
     if (nontrivial) {
+        if (DEFER) return S1_QUEUE;
         const uint32_t slot = atomicAdd(P.ctrNontrivial, 1u);
         if (slot < P.ntCap) P.nontrivial[slot] = queueEntry;
-        return;
+        return S1_NONE;
     }
 
     // per-lane incremental rasterisation (:200-269)
@@ -336,6 +352,11 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
     const float s0y = start_y - ay + 0.0f;
     float s_row = (s0x * vacy - s0y * vacx) * factor;
     float t_row = (vabx * s0y - vaby * s0x) * factor;
+    if (DEFER) {
+        *rt = RasterTri{s_row, t_row, ds_dx, ds_dy, dt_dx, dt_dy, iza, izb, izc, f2i(start_x), f2i(start_y),
+                        size_x, size_y, inRange};
+        return size_x > 0 && size_y > 0 ? S1_RASTER : S1_NONE;
+    }
     uint32_t rowPix = (uint32_t)f2i(start_x) + (uint32_t)V.W * (uint32_t)f2i(start_y);
     // The reference also tests pixelID < W*H; every sample here is inside
     // the screen (the box is clamped to [0, W-1] x [0, H-1] before ceil, and
@@ -364,6 +385,7 @@ __device__ __forceinline__ void stage1_core(const RasterParams& P, const ViewPar
         t_row += dt_dy;
         rowPix += (uint32_t)V.W;
     }
+    return S1_NONE;
 }
 
 __device__ __forceinline__ void stage1_triangle(const RasterParams& P, const ViewParams& V,
@@ -1323,6 +1345,193 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && 
             }
         }
     });
+}
+
+// ---------------------------------------------------------------------------
+// Stage 1 of draws whose triangles cover several samples each
+// (k_stage1_coarse): at most kCoarseTrisPerPixel triangles per pixel of the
+// target.  Such a draw is bound by its rasterisation, not by its geometry:
+// by the 64-bit atomics (a 1 M-triangle sphere filling 1080p issues 1.75 M,
+// at the 27 G/s that HBM takes scattered ones) and, when it has few
+// triangles, by the per-lane walk of one triangle's box on a chip that is
+// otherwise idle.
+//  * Waves take their minima in an LDS tile (raster_wave) and send the tile's
+//    covered samples row by row.
+//  * 2^splitShift neighbouring lanes share a triangle and draw its box rows in
+//    turn, as long as the draw's lanes fit the chip at once.
+//  * The stage-2 entries of a workgroup are appended with one atomic.
+// One triangle per lane group and no prefetch across batches: the waves of a
+// CU hide each other's latency (with s1_sweep's prefetch, which holds 71
+// VGPRs against 60, the 1 M sphere took 68 us against 60).
+// Measured against k_stage1, stage 1 of spheres: 1 M triangles 1080p 60
+// against 95 us; 32 K triangles 1080p 18 against 60 and 4K 26 against 71; 2 K
+// triangles 1080p 13 against 60 (a wave of k_stage1 walked 64 boxes of up to
+// 128 samples with most of the chip idle).
+// ---------------------------------------------------------------------------
+
+constexpr uint32_t kTilePixels = 512;      // LDS samples per wave (4 KB)
+constexpr uint32_t kTileMinLanes = 24;     // drawing lanes from which the tile pays for its clear and flush
+
+namespace {
+
+// Draws rows slot, slot + step, ... of the lane's triangle (the reference's
+// loop :200-269; the row increments are added one by one, as there).
+// `pix` is the address of the box's first sample, counted by emit's unit, and
+// rowStep that of a row.  The reference also tests pixelID < W*H; every
+// sample here is inside the screen (the box is clamped to [0, W-1] x
+// [0, H-1] before ceil, and a NaN bound clamps to an edge), so that test is
+// always true.
+template <typename Emit>
+__device__ __forceinline__ void raster_rows(const RasterTri& r, bool fast, uint64_t id, uint32_t slot, uint32_t step,
+                                            uint32_t pix, uint32_t rowStep, Emit&& emit) {
+    float s_row = r.s, t_row = r.t;
+    for (uint32_t q = 0; q < slot; q++) {
+        s_row += r.ds_dy;
+        t_row += r.dt_dy;
+    }
+    for (int32_t y = (int32_t)slot; y < r.h; y += (int32_t)step) {
+        float s = s_row, t = t_row;
+        uint32_t at = pix + (uint32_t)y * rowStep;
+        for (int32_t x = 0; x < r.w; x++) {
+            const float v = 1.0f - (s + t);
+            if (s > 0.0f && t > 0.0f && v > 0.0f) {
+                const float inv_depth = (v * r.iza + s * r.izb) + t * r.izc;
+                uint64_t packed;
+                if (fast) {   // wave-uniform branch: a finite depth, no infinity to map
+                    const uint32_t bits = __builtin_bit_cast(uint32_t, rcp_refined(inv_depth)) & 0x7FFFFFF8u;
+                    packed = ((uint64_t)bits << 33) | id;
+                } else {
+                    packed = pack_pixel(1.0f / inv_depth, id);
+                }
+                emit(at, packed);
+            }
+            s += r.ds_dx;
+            t += r.dt_dx;
+            at++;
+        }
+        for (uint32_t q = 0; q < step; q++) {
+            s_row += r.ds_dy;
+            t_row += r.dt_dy;
+        }
+    }
+}
+
+// Rasterises the wave's triangles (lanes with `has`); every lane of the wave
+// calls it.  Neighbouring triangles touch neighbouring samples, and an
+// atomicMin to HBM costs per cache line that an instruction touches (27 G
+// scattered lanes/s against 206 G/s when 64 lanes hit 512 contiguous bytes).
+// So when enough lanes draw and their common box fits the wave's LDS tile,
+// the wave takes the minima there first; the minimum of minima is the same
+// value.
+__device__ __forceinline__ void raster_wave(const ViewParams& V, uint64_t* tile, const RasterTri& r, bool has,
+                                            uint64_t id, uint32_t slot, uint32_t step) {
+    const uint64_t drawn = __ballot(has);
+    if (drawn == 0ull) return;
+    const bool fast = __ballot(has && !r.fast) == 0ull;
+    if ((uint32_t)__popcll(drawn) >= kTileMinLanes) {
+        const int32_t x0 = wave_min_i(has ? r.x : 0x7FFFFFFF), x1 = wave_max_i(has ? r.x + r.w : -1);
+        const int32_t y0 = wave_min_i(has ? r.y : 0x7FFFFFFF), y1 = wave_max_i(has ? r.y + r.h : -1);
+        const uint32_t bw = (uint32_t)(x1 - x0), bh = (uint32_t)(y1 - y0);
+        // the tile's width is a power of two of at least 16 samples (one 128-byte line)
+        const uint32_t lg = bw <= 16u ? 4u : 32u - (uint32_t)__builtin_clz(bw - 1u);
+        if (bw <= kTilePixels && bh <= (kTilePixels >> lg)) {
+            const uint32_t lane = threadIdx.x & (kWave - 1);
+            const uint32_t count = bh << lg;
+            for (uint32_t k = lane; k < count; k += kWave) tile[k] = ~0ull;
+            wave_sync();
+            if (has)
+                raster_rows(r, fast, id, slot, step, ((uint32_t)(r.y - y0) << lg) + (uint32_t)(r.x - x0), 1u << lg,
+                            [&](uint32_t at, uint64_t packed) {
+                                atomicMin((unsigned long long*)(tile + at), (unsigned long long)packed);
+                            });
+            wave_sync();
+            const uint32_t origin = (uint32_t)x0 + (uint32_t)V.W * (uint32_t)y0;
+            for (uint32_t k = lane; k < count; k += kWave) {
+                const uint64_t v = tile[k];
+                if (v != ~0ull)
+                    atomic_min_fb(V.fb, origin + (k & ((1u << lg) - 1u)) + (uint32_t)V.W * (k >> lg), v);
+            }
+            wave_sync();
+            return;
+        }
+    }
+    if (has)
+        raster_rows(r, fast, id, slot, step, (uint32_t)r.x + (uint32_t)V.W * (uint32_t)r.y, (uint32_t)V.W,
+                    [&](uint32_t at, uint64_t packed) { atomic_min_fb(V.fb, at, packed); });
+}
+
+}  // namespace
+
+template <bool PU16>
+__global__ __launch_bounds__(256) void k_stage1_coarse(RasterParams P) {
+    __shared__ uint64_t tiles[256 / kWave][kTilePixels];
+    __shared__ uint32_t queued[256 / kWave], queueBase;
+    uint64_t* tile = tiles[threadIdx.x / kWave];
+    const ViewParams V0 = kconst(P.views)[0];
+    const auto transforms = kconst(V0.transforms);
+    const uint32_t shift = P.splitShift;
+    const uint32_t slot = threadIdx.x & ((1u << shift) - 1u), step = 1u << shift;
+    const uint32_t numBatches = P.numBatches;
+    for (uint32_t batch = blockIdx.x; batch < numBatches; batch += gridDim.x) {
+        const S1Item it = s1_item(P, find_item(P, batch), numBatches);
+        const uint32_t tri = ((batch - it.firstBatch) << P.batchShift) + (threadIdx.x >> shift);
+        const uint32_t t = min(tri, it.numTriangles - 1u);
+        f3 A, B, C;
+        if constexpr (PU16) {
+            const float cf[3] = {it.cfx, it.cfy, it.cfz}, mn[3] = {it.mnx, it.mny, it.mnz};
+            const uint64_t off = (uint64_t)it.bits * (3ull * t);
+            A = load_pos_pu16(it.positions, bit_read(it.indices, off, it.bits) + it.indexMin, cf, mn);
+            B = load_pos_pu16(it.positions, bit_read(it.indices, off + it.bits, it.bits) + it.indexMin, cf, mn);
+            C = load_pos_pu16(it.positions, bit_read(it.indices, off + 2u * it.bits, it.bits) + it.indexMin, cf, mn);
+        } else {
+            uint32_t i0, i1, i2;
+            s1_indices(it, t, i0, i1, i2);
+            A = load_pos_g(it.positions, i0);
+            B = load_pos_g(it.positions, i1);
+            C = load_pos_g(it.positions, i2);
+        }
+        const uint32_t cullOrder = item_cull_order(P, it.instCount);
+        for (uint32_t j = 0; j < it.instCount; j++) {
+            const uint32_t inst = it.instOffset + j;
+            const auto T = transforms + inst;
+            float m[16];
+            #pragma unroll
+            for (int e = 0; e < 16; e++) m[e] = T->m[e];
+            const uint64_t id = it.cumm + (uint64_t)tri + (uint64_t)(j * it.numTriangles);
+            RasterTri rt;
+            S1Result todo = S1_NONE;
+            const uint64_t entry = ((uint64_t)inst << 32) | (uint64_t)tri;
+            if (tri < it.numTriangles) {
+                VQ qa{}, qb{}, qc{};
+                qa.d = -xform_row(m, 2, A);
+                qb.d = -xform_row(m, 2, B);
+                qc.d = -xform_row(m, 2, C);
+                todo = stage1_core<false, true>(P, V0, m, T->flip != 0u, A, B, C, qa, qb, qc, id, entry, cullOrder,
+                                                &rt);
+            }
+            // the stage-2 entries of the workgroup, appended with one atomic
+            // (each returning atomic on the one counter takes 6 ns)
+            const bool append = todo == S1_QUEUE && slot == 0u;
+            const uint64_t appending = __ballot(append);
+            __syncthreads();   // the previous round's base has been read
+            if ((threadIdx.x & (kWave - 1)) == 0) queued[threadIdx.x / kWave] = (uint32_t)__popcll(appending);
+            __syncthreads();
+            uint32_t before = 0, total = 0;
+            #pragma unroll
+            for (uint32_t w = 0; w < 256 / kWave; w++) {
+                if (w < threadIdx.x / kWave) before += queued[w];
+                total += queued[w];
+            }
+            if (total > 0) {   // the same in every thread
+                if (threadIdx.x == 0) queueBase = atomicAdd(P.ctrNontrivial, total);
+                __syncthreads();
+                const uint32_t at = queueBase + before + __builtin_amdgcn_mbcnt_hi((uint32_t)(appending >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)appending, 0u));
+                if (append && at < P.ntCap) P.nontrivial[at] = entry;
+            }
+            raster_wave(V0, tile, rt, todo == S1_RASTER && (int32_t)slot < rt.h, id, slot, step);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2814,6 +3023,12 @@ hipError_t launch_s1_any(const RasterParams& P, uint32_t block, uint32_t k, uint
 hipError_t launch_stage1(const RasterParams& P, uint32_t block, uint32_t trisPerLane, uint32_t grid, bool pu16,
                          bool instanceBoxes, hipStream_t stream) {
     return launch_s1_any(P, block, trisPerLane, grid, pu16, false, instanceBoxes, stream);
+}
+
+hipError_t launch_stage1_coarse(const RasterParams& P, uint32_t grid, bool pu16, hipStream_t stream) {
+    if (pu16) hipLaunchKernelGGL(k_stage1_coarse<true>, dim3(grid), dim3(256), 0, stream, P);
+    else hipLaunchKernelGGL(k_stage1_coarse<false>, dim3(grid), dim3(256), 0, stream, P);
+    return hipGetLastError();
 }
 
 hipError_t launch_stage1_pairs(const RasterParams& P, uint32_t block, uint32_t grid, bool pu16, hipStream_t stream) {

@@ -230,7 +230,8 @@ typedef struct crx_draw_stats {
     uint32_t num_huge;             /* tile entries in the stage-3 queue */
     uint32_t redraws;              /* redraws caused by queue growth */
     uint32_t stage1_kernel;        /* the stage-1 kernel the draw ran: 0 = k_stage1 (lanes take
-                                      triangles a block apart), 1 = k_stage1_views (several views),
+                                      triangles a block apart) or, for draws of few triangles per
+                                      pixel, k_stage1_coarse, 1 = k_stage1_views (several views),
                                       2 = k_stage1_pairs (consecutive pairs, tuning.stage1_layout) */
 } crx_draw_stats;
 
