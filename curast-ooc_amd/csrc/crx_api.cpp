@@ -222,6 +222,7 @@ void set_counter_block(RasterParams& P, uint32_t* block) {
     P.cursor2 = block + CTR_CURSOR2;
     P.cursor3 = block + CTR_CURSOR3;
     P.claims = block + CTR_CLAIM;
+    P.unitCount = block + CTR_UNITS;
 }
 
 // Per-view record of a draw: size, projection and the view's transforms.
@@ -298,12 +299,34 @@ uint32_t detect_row_triangles(const uint32_t* idx, uint64_t T) {
     return (uint32_t)best & ~1u;
 }
 
+// Pair layout (batches of one wave's 128 triangles): units of stripRows rows
+// of a strip of stripBatches batches of the mesh's rows (a mesh stored in
+// rows of at least eight batches), else of rows of 128 triangles (a
+// contiguous walk).
+uint64_t pair_layout(DrawItem& it, uint32_t rowHint, uint32_t stripRows, uint32_t stripBatches) {
+    constexpr uint64_t waveTris = 128;
+    const bool strips = rowHint >= 8 * waveTris;
+    const uint64_t stripTris = waveTris * (strips ? stripBatches : 1u);
+    it.rowTris = strips ? rowHint : (uint32_t)waveTris;
+    it.unitCols = strips ? stripBatches : 1u;
+    it.strips = strips ? (uint32_t)((rowHint + stripTris - 1) / stripTris) : 1u;
+    it.unitRows = stripRows;
+    const uint64_t rows = ((uint64_t)it.numTriangles + it.rowTris - 1) / it.rowTris;
+    it.unitSegs = (uint32_t)((rows + it.unitRows - 1) / it.unitRows);
+    // the groups of a strip rounded up to a multiple of 8 (the units past
+    // the last row are empty): unit s * unitSegs + g then runs on the XCD
+    // of its group g for every strip s, so the waves that draw the two
+    // sides of a strip edge share their XCD's L2
+    if (strips) it.unitSegs = (it.unitSegs + 7u) & ~7u;
+    return (uint64_t)it.strips * it.unitSegs;
+}
+
 // Host records and metadata layout of a draw of numViews >= 1 views sharing
 // one instance list (transforms view-major).  No device work.
 crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMeshes, const crx_cmesh* instances,
                      uint32_t numInstances, const crx_mat4* transforms, const crx_render_target* targets,
                      uint32_t numViews, int instanced, const uint8_t* skip, DrawPlan* plan, bool instUnchanged,
-                     bool prefix) {
+                     bool prefix, const DrawBounds& bounds) {
     if (!ctx) return fail(CRX_INVALID_ARG, "ctx is NULL");
     if (numViews == 0 || numViews > kMaxViews)
         return fail(CRX_INVALID_ARG, "numViews must be in [1, " + std::to_string(kMaxViews) + "]");
@@ -360,7 +383,6 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
                                (D.block / 64);
         D.runs = tris >= 16ull * 128ull * waves;
     }
-
     // few triangles per pixel: each covers several samples, and the draw is
     // bound by its rasterisation (k_stage1_coarse).  The tuning's knobs of
     // the other kernels (an explicit block, triangles per lane or walk) keep it off.
@@ -379,6 +401,16 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
             D.batchShift = 8u - D.splitShift;
         }
     }
+    // A draw of meshes whose units have boxes draws only the units the view
+    // may see.  The boxes are those of the default walk.
+    if (bounds.boxes && !D.coarse && numViews == 1 && !manyInstances && D.block == 256 && tu.stage1_tris_per_lane == 0 &&
+        tu.stage1_layout == 2 && tu.stage1_strip_rows == kUnitRows && tu.stage1_strip_batches == 1) {
+        uint64_t tris = 0;
+        for (uint32_t k = 0; k < D.numItems; k++) tris += bounds.boxes[k] ? list[k].numTriangles : 0u;
+        D.listed = bounds.always || tris >= kListMinTris;
+        if (D.listed) D.runs = true;
+    }
+
     const uint64_t batchTris = 1ull << D.batchShift;
 
     D.items.resize(D.numItems);
@@ -410,28 +442,12 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
         it.cf[0] = m.compressionFactor.x; it.cf[1] = m.compressionFactor.y; it.cf[2] = m.compressionFactor.z;
         it.amin[0] = m.aabb.min.x; it.amin[1] = m.aabb.min.y; it.amin[2] = m.aabb.min.z;
         it.numVertices = m.numVertices;
-        // pair layout (batches of one wave's 128 triangles): units of
-        // stage1_strip_rows rows of a strip of stage1_strip_batches batches
-        // of the mesh's rows (a mesh stored in rows of at least eight
-        // batches), else of rows of 128 triangles (a contiguous walk)
-        constexpr uint64_t waveTris = 128;
         const uint32_t rowHint = (D.runs && tu.stage1_layout == 2) ? row_hint_of(m.indices) : 0u;
-        const bool strips = rowHint >= 8 * waveTris;
-        const uint64_t stripTris = waveTris * (strips ? tu.stage1_strip_batches : 1u);
-        it.rowTris = strips ? rowHint : (uint32_t)waveTris;
-        it.unitCols = strips ? tu.stage1_strip_batches : 1u;
-        it.strips = strips ? (uint32_t)((rowHint + stripTris - 1) / stripTris) : 1u;
-        it.unitRows = tu.stage1_strip_rows;
-        const uint64_t rows = ((uint64_t)m.numTriangles + it.rowTris - 1) / it.rowTris;
-        it.unitSegs = (uint32_t)((rows + it.unitRows - 1) / it.unitRows);
-        // the groups of a strip rounded up to a multiple of 8 (the units past
-        // the last row are empty): unit s * unitSegs + g then runs on the XCD
-        // of its group g for every strip s, so the waves that draw the two
-        // sides of a strip edge share their XCD's L2
-        if (strips) it.unitSegs = (it.unitSegs + 7u) & ~7u;
-        const uint64_t units = (uint64_t)it.strips * it.unitSegs;
+        const uint64_t units = pair_layout(it, rowHint, tu.stage1_strip_rows, tu.stage1_strip_batches);
+        if (D.listed) it.bounds = bounds.boxes[k];
         D.batches += D.runs ? units : ((uint64_t)m.numTriangles + batchTris - 1) >> D.batchShift;
         D.tris += (uint64_t)m.numTriangles * (uint64_t)cnt;
+        if (D.listed && D.batches >= (1ull << 31)) return fail(CRX_INVALID_ARG, "too many triangle batches for one draw");
         if (D.batches >= (1ull << 32)) return fail(CRX_INVALID_ARG, "too many triangle batches for one draw");
     }
     // instUnchanged: the list is the one the plan's records were built (and
@@ -464,7 +480,7 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
     if (sched.wavesPerCU == 0 || D.coarse) {   // one workgroup per batch
         D.g1 = (uint32_t)std::min<uint64_t>(D.batches, 1ull << 31);
     } else {
-        D.g1 = grid_for(ctx, sched.wavesPerCU, D.block / 64);
+        D.g1 = D.listed ? (uint32_t)ctx->numCUs * 10u : grid_for(ctx, sched.wavesPerCU, D.block / 64);
         if (D.g1 > D.batches) D.g1 = (uint32_t)D.batches;
     }
     D.g1 = (D.g1 + 7u) & ~7u;   // the stage-1 XCD split assumes a multiple of 8 workgroups
@@ -530,7 +546,10 @@ hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& D, const RasterParam
     }
     record(ctx, T_S1, stream);
     if (D.numViews == 1 && !viewsKernel && D.runs)
-        e = launch_stage1_pairs(P, D.block, D.g1, D.pu16, stream);
+    {
+        if (D.listed) e = launch_cull_units(P, stream);
+        if (e == hipSuccess) e = launch_stage1_pairs(P, D.block, D.g1, D.pu16, D.listed, stream);
+    }
     else if (D.numViews == 1 && !viewsKernel && D.coarse)
         e = launch_stage1_coarse(P, D.g1, D.pu16, stream);
     else if (D.numViews == 1 && !viewsKernel)
@@ -576,7 +595,7 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
     const bool sameLists = ex.listsKey != 0 && ex.listsKey == ctx->metaListsKey;
     ctx->metaListsKey = 0;
     CRX_TRY(plan_draw(ctx, meshes, numMeshes, instances, numInstances, transforms, targets, numViews, instanced,
-                      ex.skip, &D, sameLists, ex.prefix));
+                      ex.skip, &D, sameLists, ex.prefix, ex.bounds));
     if (stats) stats->num_triangles = D.tris * numViews;
     if (D.batches == 0 && !ex.afterStages) return CRX_OK;
     CRX_HIP(hipSetDevice(ctx->device));
@@ -625,6 +644,8 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
         return finish();
     }
     CRX_TRY(ensure_queues(ctx, ctx->tuning.max_nontrivial, ctx->tuning.max_huge));
+    if (D.listed) CRX_TRY(ctx->unitList.reserve(D.batches * sizeof(uint32_t)));
+    P.units = static_cast<uint32_t*>(ctx->unitList.ptr);
 
     uint32_t redraws = 0;
     for (;;) {
@@ -987,6 +1008,8 @@ uint32_t scene_lists(crx_scene* scene, const crx_view* views, uint32_t numViews,
         scene->instances.resize(n);
         scene->prefix.resize(n);
         scene->nodeOf.resize(n);
+        scene->uniqueBounds.resize(n);
+        scene->instanceBounds.resize(n);
         uint64_t sum = 0;
         uint32_t u = 0;
         for (uint32_t i = 0; i < n; i++) {
@@ -1019,8 +1042,10 @@ uint32_t scene_lists(crx_scene* scene, const crx_view* views, uint32_t numViews,
             scene->nodeOf[i] = kept[i];
             sum += cm.numTriangles;
             scene->instances[i] = cm;
+            scene->instanceBounds[i] = nd.mesh->shared ? nullptr : nd.mesh->bounds;
             if (u == 0 || scene->unique[u - 1].address != cm.address || !settings.instanced) {
                 scene->unique[u] = cm;
+                scene->uniqueBounds[u] = scene->instanceBounds[i];
                 u++;
             }
             scene->unique[u - 1].instances.count++;
@@ -1129,6 +1154,7 @@ crx_status render_views(crx_context* ctx, crx_scene* scene, const crx_view* view
     ex.prefix = settings.resolve != 0;
     ex.earlyReturn = true;
     ex.countersZeroed = zeroed;
+    ex.bounds.boxes = settings.instanced ? scene->uniqueBounds.data() : scene->instanceBounds.data();
     CRX_TRY(draw_views(ctx, scene->unique.data(), u, scene->instances.data(), n, scene->transforms.data(),
                        targets.data(), numViews, settings.instanced, stream, stats, ex));
     return CRX_OK;
@@ -1223,6 +1249,7 @@ crx_status crx_context_destroy(crx_context* ctx) {
     ctx->drawMeta.release();
     ctx->resolveMeta.release();
     ctx->clearMeta.release();
+    ctx->unitList.release();
     ctx->argsMeta.release();
     if (ctx->argsUse) (void)hipEventDestroy(ctx->argsUse);
     if (ctx->ctr) (void)hipFree(ctx->ctr);
@@ -1534,6 +1561,38 @@ void crx_mat4_mul(const crx_mat4* a, const crx_mat4* b, crx_mat4* out) {
 
 // ---- scene API --------------------------------------------------------------
 
+namespace {
+
+// The boxes of a new mesh's units, from its own device geometry.  A draw
+// without boxes is the same draw, so a failed allocation only leaves them out.
+crx_status mesh_bounds(crx_mesh* m) {
+    if (m->numTriangles < kListMinTris || !m->positions) return CRX_OK;
+    DrawItem it{};
+    it.indices = m->indices ? m->indices : reinterpret_cast<const uint32_t*>(m->positions);
+    it.indexMask = m->indices ? 0xFFFFFFFFu : 0u;
+    it.positions = m->positions;
+    it.numTriangles = m->numTriangles;
+    it.bitsPerIndex = m->bitsPerIndex;
+    it.indexMin = m->indexMin;
+    it.cf[0] = m->compressionFactor.x; it.cf[1] = m->compressionFactor.y; it.cf[2] = m->compressionFactor.z;
+    it.amin[0] = m->aabb.min.x; it.amin[1] = m->aabb.min.y; it.amin[2] = m->aabb.min.z;
+    it.numVertices = m->numVertices;
+    const uint64_t units = pair_layout(it, m->rowTris, kUnitRows, 1u);
+    if (units >= (1ull << 31)) return CRX_OK;
+    if (hipMalloc((void**)&m->bounds, units * sizeof(UnitBox)) != hipSuccess) {
+        (void)hipGetLastError();
+        m->bounds = nullptr;
+        return CRX_OK;
+    }
+    hipError_t e = launch_unit_bounds(it, m->compressed, (uint32_t)units, m->bounds, nullptr);
+    // frames on any stream may use the mesh as soon as it is returned
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) return fail(CRX_HIP_ERROR, std::string("mesh bounds: ") + hipGetErrorString(e));
+    return CRX_OK;
+}
+
+}  // namespace
+
 crx_status crx_mesh_create(crx_context* ctx, const float* positions, uint32_t numVertices,
                            const uint32_t* indices, uint32_t numTriangles, const uint32_t* colors,
                            crx_mesh** out) {
@@ -1584,6 +1643,11 @@ crx_status crx_mesh_create(crx_context* ctx, const float* positions, uint32_t nu
             std::lock_guard<std::mutex> lk(g_rowHintsMu);
             g_rowHints[m->indices] = m->rowTris;
         }
+    }
+    const crx_status bs = mesh_bounds(m);
+    if (bs != CRX_OK) {
+        crx_mesh_destroy(m);
+        return bs;
     }
     *out = m;
     return CRX_OK;
@@ -1704,6 +1768,11 @@ crx_status crx_mesh_create_compressed(crx_context* ctx, const float* positions, 
             g_rowHints[m->indices] = m->rowTris;
         }
     }
+    const crx_status bs = mesh_bounds(m);
+    if (bs != CRX_OK) {
+        crx_mesh_destroy(m);
+        return bs;
+    }
     *out = m;
     return CRX_OK;
 }
@@ -1740,6 +1809,7 @@ crx_status crx_mesh_destroy(crx_mesh* mesh) {
         if (mesh->indices) (void)hipFree(mesh->indices);
         if (mesh->colors) (void)hipFree(mesh->colors);
     }
+    if (mesh->bounds) (void)hipFree(mesh->bounds);
     if (mesh->uvs) (void)hipFree(mesh->uvs);
     if (mesh->normals) (void)hipFree(mesh->normals);
     delete mesh;
@@ -1794,6 +1864,11 @@ crx_status crx_mesh_buffers(const crx_mesh* mesh, const float** d_positions, con
     if (d_positions) *d_positions = mesh->positions;
     if (d_indices) *d_indices = mesh->indices;
     if (d_colors) *d_colors = mesh->colors;
+    // whoever holds the addresses may write there: the boxes no longer count
+    if (!mesh->shared) {
+        mesh->shared = true;
+        mesh->ctx->attrEpoch++;
+    }
     return CRX_OK;
 }
 

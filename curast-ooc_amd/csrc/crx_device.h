@@ -15,6 +15,22 @@
 
 namespace crx {
 
+// Object-space box of the triangles of one stage-1 unit of a mesh, with the
+// largest coordinate magnitude M in it.  A unit that holds a NaN or infinite
+// coordinate has M = +inf (and no box).  An empty unit has lo > hi.
+struct UnitBox {
+    float lo[3], hi[3];
+    float M;
+    uint32_t pad;
+};
+
+// Rows per unit of a mesh's boxes: those of the default walk
+// (crx_tuning::stage1_strip_rows), at 128 triangles (one wave) per row.
+constexpr uint32_t kUnitRows = 8;
+
+// Triangles from which a mesh gets unit boxes and a draw uses them.
+constexpr uint64_t kListMinTris = 1u << 20;
+
 // Stage-1 work unit.  Instanced draws: one unit per unique mesh that loops
 // over instCount consecutive instances.  Non-instanced draws: one unit per
 // instance (instCount == 1).
@@ -45,6 +61,9 @@ struct DrawItem {
     uint32_t unitRows;
     uint32_t unitSegs;
     uint32_t unitCols;
+    // Boxes of the item's units (unit u of the item: bounds[u - firstBatch]),
+    // or null: none known, every unit is drawn.
+    const UnitBox* bounds;
 };
 
 // Per-instance record for stage 2, stage 3 and resolve.
@@ -92,6 +111,7 @@ enum Counter : int {
     CTR_HUGE = 1,         // stage-3 tile entries produced by stage 2
     CTR_CURSOR2 = 2,      // stage-2 work cursor
     CTR_CURSOR3 = 3,      // stage-3 work cursor
+    CTR_UNITS = 4,        // units k_cull_units listed
     // k_stage1_pairs: eight unit counters, one per XCD, each on its own
     // 128-byte line (word CTR_CLAIM + kClaimStride * xcd)
     CTR_CLAIM = 32,
@@ -160,6 +180,8 @@ struct RasterParams {
     uint32_t numWaves2;      // waves in the stage-2 grid
     uint32_t numWaves3;      // waves in the stage-3 grid
     uint32_t splitShift;     // k_stage1_coarse: log2(lanes per triangle)
+    uint32_t* units;         // k_cull_units: the units left to draw ...
+    uint32_t* unitCount;     // ... and their number (CTR_UNITS)
     uint32_t* claims;        // k_stage1_pairs: the per-XCD unit counters (CTR_CLAIM of the counter block)
 };
 

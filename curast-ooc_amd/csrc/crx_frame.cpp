@@ -32,7 +32,8 @@ struct crx_frame {
 
     DrawPlan plan;
     size_t nodes = 0;                 // scene node count at creation
-    DeviceBuffer drawMeta, resolveMeta, clearMeta, nontrivial, huge;
+    uint64_t attrEpoch = 0;           // the context's attrEpoch the records were written at
+    DeviceBuffer drawMeta, resolveMeta, clearMeta, nontrivial, huge, unitList;
     uint32_t ntCap = 0, hugeCap = 0;
     uint32_t* ctr = nullptr;          // device counters
     uint32_t* ctrHost = nullptr;      // page-locked copy written by the graph
@@ -67,9 +68,13 @@ crx_status frame_fill(crx_frame* F, bool write) {
     view_targets(F->views.data(), F->numViews, F->fbs.data(), F->cbs.data(), F->settings.resolve != 0, &targets,
                  &clearBufs, &clearPx);
     DrawPlan D;
+    DrawBounds bounds;
+    bounds.boxes = F->settings.instanced ? sc->uniqueBounds.data() : sc->instanceBounds.data();
+    bounds.always = write && F->plan.listed;
     CRX_TRY(plan_draw(F->ctx, sc->unique.data(), u, sc->instances.data(), n, sc->transforms.data(), targets.data(),
                       F->numViews, F->settings.instanced, F->settings.frustum_culling ? sc->skip.data() : nullptr,
-                      &D));
+                      &D, false, false, bounds));
+    F->attrEpoch = F->ctx->attrEpoch;
     std::vector<char> rimage;
     size_t offViews = 0;
     uint32_t rblocks = 0;
@@ -101,6 +106,7 @@ crx_status frame_fill(crx_frame* F, bool write) {
     F->P.huge = static_cast<int4*>(F->huge.ptr);
     F->P.ntCap = F->ntCap;
     F->P.hugeCap = F->hugeCap;
+    F->P.units = static_cast<uint32_t*>(F->unitList.ptr);
     if (!rimage.empty()) std::memcpy(F->stageResolve, rimage.data(), rimage.size());
     if (!cv.empty()) std::memcpy(F->stageClear, cv.data(), F->clearBytes);
     return CRX_OK;
@@ -160,6 +166,7 @@ crx_status crx_frame_destroy(crx_frame* F) {
     F->clearMeta.release();
     F->nontrivial.release();
     F->huge.release();
+    F->unitList.release();
     if (F->ctr) (void)hipFree(F->ctr);
     if (F->ctrHost) (void)hipHostFree(F->ctrHost);
     if (F->stageDraw) (void)hipHostFree(F->stageDraw);
@@ -208,6 +215,7 @@ crx_status crx_frame_create(crx_context* ctx, crx_scene* scene, const crx_view* 
         F->hugeCap = ctx->tuning.max_huge;
         st = F->nontrivial.reserve((size_t)F->ntCap * sizeof(uint64_t));
         if (st == CRX_OK) st = F->huge.reserve((size_t)F->hugeCap * sizeof(int4));
+        if (st == CRX_OK && F->plan.listed) st = F->unitList.reserve(F->plan.batches * sizeof(uint32_t));
     }
     hip(hipMalloc(&F->ctr, CTR_COUNT * sizeof(uint32_t)), "hipMalloc");
     hip(hipHostMalloc((void**)&F->ctrHost, CTR_COUNT * sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc");
@@ -241,6 +249,11 @@ crx_status crx_frame_set_views(crx_frame* F, const crx_view* views) {
 crx_status crx_frame_launch(crx_frame* F, void* stream) {
     if (!F) return fail(CRX_INVALID_ARG, "frame is NULL");
     CRX_HIP(hipSetDevice(F->ctx->device));
+    if (F->plan.listed && F->attrEpoch != F->ctx->attrEpoch) {
+        // a mesh may have lost its boxes (crx_mesh_buffers): write the records again
+        if (F->launched) CRX_HIP(hipEventSynchronize(F->done));
+        CRX_TRY(frame_fill(F, true));
+    }
     CRX_HIP(hipGraphLaunch(F->exec, as_stream(stream)));
     CRX_HIP(hipEventRecord(F->done, as_stream(stream)));
     F->launched = true;

@@ -126,10 +126,19 @@ struct DrawPlan {
     uint32_t block = 256, trisPerLane = 1, batchShift = 8, g1 = 0, g2 = 0, g3 = 0;
     bool instanceBoxes = false;   // some item loops over >= 4 instances
     bool runs = false;            // k_stage1_runs (items carry the run layout; batches counts its units)
+    bool listed = false;          // runs over the units k_cull_units lists (some item has boxes)
     bool coarse = false;          // k_stage1_coarse (few triangles per pixel)
     uint32_t splitShift = 0;      // its lanes per triangle (log2)
     bool prefix = false;          // the image carries the instances' triangle prefix (InstanceRec::cumm)
     size_t offItems = 0, offInst = 0, offPrefix = 0, offViews = 0, offXf = 0, metaBytes = 0;
+};
+
+// Per draw item: the boxes of its mesh's units (crx_mesh::bounds), or null.
+// always: list the units whatever the items' boxes (a recorded frame keeps
+// its layout when a mesh loses them).
+struct DrawBounds {
+    const UnitBox* const* boxes = nullptr;
+    bool always = false;
 };
 
 // What a caller adds to a draw.  listsKey != 0 names the content of the
@@ -148,6 +157,7 @@ struct DrawExtras {
     bool prefix = false;
     bool earlyReturn = false;
     bool countersZeroed = false;
+    DrawBounds bounds;
 };
 
 // A hierarchy over ranges of consecutive nodes (a binary tree whose leaves
@@ -185,6 +195,7 @@ struct crx_context {
     crx::DeviceBuffer drawMeta;            // items | instances | transforms
     crx::DeviceBuffer resolveMeta;         // instances | prefix | per-view records
     crx::DeviceBuffer clearMeta;           // per-buffer clear records
+    crx::DeviceBuffer unitList;            // k_cull_units: unit numbers
     crx::Staging drawStaging, resolveStaging, clearStaging;
     // instance records (and prefix) that drawMeta holds: the list key they
     // were uploaded under (0 = none), the buffer and their byte range
@@ -200,7 +211,7 @@ struct crx_context {
     hipEvent_t ev[crx::T_COUNT] = {};
     bool recorded[crx::T_COUNT] = {};
     uint64_t meshSeq = 0;
-    uint64_t attrEpoch = 0;           // bumped by every crx_mesh_set_attributes on this context
+    uint64_t attrEpoch = 0;           // bumped by every crx_mesh_set_attributes (and mesh's loss of its boxes)
     // kernel-level entry points: the records buffer every crx_raster_stage*
     // call rebuilds its records in, and the event after the last call's
     // launches (a call on another stream waits for it)
@@ -225,6 +236,11 @@ struct crx_mesh {
     uint32_t bitsPerIndex = 0, indexMin = 0, indexMax = 0;
     crx_vec3 compressionFactor{};
     uint32_t rowTris = 0;             // triangles per row of a mesh stored in rows (0 = none found)
+    // Boxes of the mesh's units in the default walk (plan_draw's pair layout),
+    // made with the mesh from the geometry it owns; null for small meshes and
+    // once crx_mesh_buffers has handed the geometry out.
+    crx::UnitBox* bounds = nullptr;
+    mutable bool shared = false;      // crx_mesh_buffers was called
     // resolve-only vertex attributes, always owned by the mesh (crx_mesh_set_attributes)
     float* uvs = nullptr;             // 2 floats per vertex
     float* normals = nullptr;         // 3 floats per vertex
@@ -241,6 +257,7 @@ struct crx_scene {
     std::vector<Node> nodes;
     // frame-preparation scratch, kept across frames like the reference's statics
     std::vector<crx_cmesh> unique, instances;
+    std::vector<const crx::UnitBox*> uniqueBounds, instanceBounds;   // crx_mesh::bounds of each entry
     std::vector<crx_mat4> transforms;
     std::vector<uint64_t> prefix;
     std::vector<uint8_t> skip;        // [view][instance]: dropped by that view's node cull
@@ -304,7 +321,9 @@ bool box_in_frustum(const float planes[16], const crx_box3& worldBox);
 crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMeshes, const crx_cmesh* instances,
                      uint32_t numInstances, const crx_mat4* transforms, const crx_render_target* targets,
                      uint32_t numViews, int instanced, const uint8_t* skip, DrawPlan* plan,
-                     bool instUnchanged = false, bool prefix = false);
+                     bool instUnchanged = false, bool prefix = false, const DrawBounds& bounds = DrawBounds{});
+// The pair layout of a mesh's units (DrawItem::rowTris ... unitCols); returns their number.
+uint64_t pair_layout(DrawItem& it, uint32_t rowHint, uint32_t stripRows, uint32_t stripBatches);
 RasterParams plan_write(crx_context* ctx, const DrawPlan& plan, char* host, char* dev, bool writeInst = true);
 hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& plan, const RasterParams& P, bool viewsKernel,
                           hipStream_t stream, bool countersZeroed = false);

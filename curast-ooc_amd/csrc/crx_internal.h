@@ -31,7 +31,15 @@ hipError_t launch_stage1(const RasterParams& P, uint32_t block, uint32_t trisPer
 hipError_t launch_stage1_coarse(const RasterParams& P, uint32_t grid, bool pu16, hipStream_t stream);
 // Pairs of consecutive triangles per lane, block 256 (k_stage1_pairs): the
 // items carry the strip layout (DrawItem::rowTris ...).
-hipError_t launch_stage1_pairs(const RasterParams& P, uint32_t block, uint32_t grid, bool pu16, hipStream_t stream);
+// listed: the units are those k_cull_units listed (P.units, P.unitCount).
+hipError_t launch_stage1_pairs(const RasterParams& P, uint32_t block, uint32_t grid, bool pu16, bool listed,
+                               hipStream_t stream);
+// Lists the units of the pair layout that the view may see (P.units,
+// P.unitCount; the counter starts at zero).
+hipError_t launch_cull_units(const RasterParams& P, hipStream_t stream);
+// Boxes of a mesh's units in the pair layout (the item's fields as plan_draw
+// fills them for one item with kUnitRows rows per unit).
+hipError_t launch_unit_bounds(const DrawItem& item, bool pu16, uint32_t numUnits, UnitBox* out, hipStream_t stream);
 hipError_t launch_stage1_views(const RasterParams& P, uint32_t block, uint32_t trisPerLane, uint32_t grid, bool pu16,
                                hipStream_t stream);
 hipError_t launch_stage2(const RasterParams& P, uint32_t grid, hipStream_t stream);

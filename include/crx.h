@@ -541,7 +541,9 @@ crx_status crx_texture_compute_mipmap(crx_context* ctx, uint32_t* data, int32_t 
  * NORMAL the normals).  Replacing an attribute waits for the device before
  * freeing the old buffer. */
 crx_status crx_mesh_set_attributes(crx_mesh* mesh, const float* uvs, const float* normals);
-/* Device pointers of the mesh buffers (colors may be NULL). */
+/* Device pointers of the mesh buffers (colors may be NULL).  From this call
+ * on, frames of the mesh no longer skip parts of it by the boxes that
+ * crx_mesh_create computed from the geometry. */
 crx_status crx_mesh_buffers(const crx_mesh* mesh, const float** d_positions, const uint32_t** d_indices,
                             const uint32_t** d_colors);
 
