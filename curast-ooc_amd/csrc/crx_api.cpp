@@ -686,8 +686,9 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
 
 // Per-view resolve record (the instance list and prefix are shared).
 ResolveParams make_resolve_params(const crx_render_target& t, const InstanceRec* inst, const uint64_t* prefix,
-                                  uint32_t numInstances, crx_display_attribute attribute) {
+                                  uint32_t numInstances, crx_display_attribute attribute, bool fresh) {
     ResolveParams R{};
+    R.fresh = fresh ? 1u : 0u;
     R.inst = inst;
     R.prefix = prefix;
     R.fb = t.framebuffer;
@@ -698,6 +699,8 @@ ResolveParams make_resolve_params(const crx_render_target& t, const InstanceRec*
     R.attribute = (int32_t)attribute;
     R.Wf = (float)t.width;
     R.Hf = (float)t.height;
+    R.WI = 1.0f / R.Wf;
+    R.HI = 1.0f / R.Hf;
     R.p00I = 1.0f / t.proj.m[0];
     R.p11I = 1.0f / t.proj.m[5];
     const crx_mat4 viewI = mat_inverse(t.view);
@@ -753,7 +756,7 @@ crx_status resolve_blocks(const crx_render_target* targets, uint32_t numViews, R
 
 crx_status resolve_image_into(const crx_cmesh* instances, uint32_t numInstances, const uint64_t* prefix,
                               const crx_render_target* targets, uint32_t numViews, crx_display_attribute attribute,
-                              char* dev, char* out, size_t* offViews, uint32_t* blocks, bool ownedOnly = false) {
+                              char* dev, char* out, size_t* offViews, uint32_t* blocks, bool ownedOnly, bool fresh) {
     CRX_TRY(check_resolve(targets, numViews, attribute));
     if (numInstances > 0 && (!instances || !prefix)) return fail(CRX_INVALID_ARG, "instances / prefix is NULL");
     size_t offPrefix = 0;
@@ -768,7 +771,7 @@ crx_status resolve_image_into(const crx_cmesh* instances, uint32_t numInstances,
     const uint64_t* prefixDev = reinterpret_cast<const uint64_t*>(dev + offPrefix);
     ResolveParams* rv = reinterpret_cast<ResolveParams*>(out + *offViews);
     for (uint32_t v = 0; v < numViews; v++) {
-        rv[v] = make_resolve_params(targets[v], instDev, prefixDev, numInstances, attribute);
+        rv[v] = make_resolve_params(targets[v], instDev, prefixDev, numInstances, attribute, fresh);
         rv[v].ownedOnly = ownedOnly ? 1u : 0u;
     }
     return resolve_blocks(targets, numViews, rv, blocks);
@@ -776,11 +779,11 @@ crx_status resolve_image_into(const crx_cmesh* instances, uint32_t numInstances,
 
 crx_status resolve_image(const crx_cmesh* instances, uint32_t numInstances, const uint64_t* prefix,
                          const crx_render_target* targets, uint32_t numViews, crx_display_attribute attribute,
-                         char* dev, std::vector<char>* image, size_t* offViews, uint32_t* blocks) {
+                         char* dev, std::vector<char>* image, size_t* offViews, uint32_t* blocks, bool fresh) {
     size_t offPrefix = 0;
     image->resize(resolve_image_layout(numInstances, numViews, &offPrefix, offViews));
     return resolve_image_into(instances, numInstances, prefix, targets, numViews, attribute, dev, image->data(),
-                              offViews, blocks);
+                              offViews, blocks, false, fresh);
 }
 
 // kernel_resolve_visbuffer_to_colorbuffer2D (resolve.cu:640-1141) for
@@ -800,7 +803,7 @@ crx_status resolve_views(crx_context* ctx, const crx_cmesh* instances, uint32_t 
     CRX_TRY(ctx->resolveStaging.acquire(bytes));
     char* image = static_cast<char*>(ctx->resolveStaging.ptr);
     CRX_TRY(resolve_image_into(instances, numInstances, prefix, targets, numViews, attribute, meta, image, &offViews,
-                               &blocks, ownedOnly));
+                               &blocks, ownedOnly, false));
     const ResolveParams* rv = reinterpret_cast<const ResolveParams*>(image + offViews);
     if (numInstances || numViews > 1) {
         CRX_HIP(hipMemcpyAsync(meta, image, bytes, hipMemcpyHostToDevice, stream));
@@ -826,7 +829,7 @@ crx_status resolve_views_device(crx_context* ctx, const InstanceRec* instDev, co
     CRX_HIP(hipSetDevice(ctx->device));
     if (numViews == 1) {
         // one view: its record is the kernel argument, nothing to upload
-        const ResolveParams R = make_resolve_params(targets[0], instDev, prefixDev, numInstances, attribute);
+        const ResolveParams R = make_resolve_params(targets[0], instDev, prefixDev, numInstances, attribute, true);
         record(ctx, T_RESOLVE, stream);
         CRX_HIP(launch_resolve(R, stream));
         record(ctx, T_RESOLVE_END, stream);
@@ -838,7 +841,7 @@ crx_status resolve_views_device(crx_context* ctx, const InstanceRec* instDev, co
     CRX_TRY(ctx->resolveStaging.acquire(bytes));
     ResolveParams* rv = static_cast<ResolveParams*>(ctx->resolveStaging.ptr);
     for (uint32_t v = 0; v < numViews; v++)
-        rv[v] = make_resolve_params(targets[v], instDev, prefixDev, numInstances, attribute);
+        rv[v] = make_resolve_params(targets[v], instDev, prefixDev, numInstances, attribute, true);
     uint32_t blocks = 0;
     CRX_TRY(resolve_blocks(targets, numViews, rv, &blocks));
     CRX_HIP(hipMemcpyAsync(ctx->resolveMeta.ptr, rv, bytes, hipMemcpyHostToDevice, stream));
@@ -1093,13 +1096,10 @@ void view_targets(const crx_view* views, uint32_t numViews, uint64_t* const* fra
         t.cameraPos = crx_vec3{cam.x, cam.y, cam.z};
         t.f = views[v].proj.m[5];
         t.aspect = (float)views[v].width / (float)views[v].height;
-        const uint32_t px = (uint32_t)views[v].width * (uint32_t)views[v].height;
+        // the resolve writes every pixel of the colour buffer without reading
+        // it (ResolveParams::fresh), so only the visibility buffer is cleared
         clearBufs->push_back(t.framebuffer);
-        clearPx->push_back(px);
-        if (resolve) {
-            clearBufs->push_back(t.colorbuffer);
-            clearPx->push_back(px);
-        }
+        clearPx->push_back((uint32_t)views[v].width * (uint32_t)views[v].height);
     }
 }
 

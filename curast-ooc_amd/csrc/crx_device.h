@@ -194,6 +194,7 @@ struct ResolveParams {
     int32_t W, H;
     int32_t attribute;
     float Wf, Hf;
+    float WI, HI;              // RN(1 / Wf), RN(1 / Hf)
     float p00I, p11I;          // 1/proj[0][0], 1/proj[1][1]
     float viewI[16];           // inverse(view), GLM order, computed once per frame
     float origin[3];           // viewI * (0,0,0,1)
@@ -202,6 +203,7 @@ struct ResolveParams {
     uint32_t firstBlock;       // multi-view resolve: first 64x4 tile block of this view
     uint32_t ownedOnly;        // 1: leave pixels whose triangle is not in the listed instances
                                // (a resolve in passes over groups of instances)
+    uint32_t fresh;            // 1: the colour buffer counts as cleared (it is neither cleared nor read)
 };
 
 // The five stage counters of the kernel-level entry points (RasterArgs:

@@ -81,7 +81,7 @@ crx_status frame_fill(crx_frame* F, bool write) {
     if (F->settings.resolve) {
         CRX_TRY(resolve_image(sc->instances.data(), n, sc->prefix.data(), targets.data(), F->numViews,
                               (crx_display_attribute)F->settings.attribute,
-                              static_cast<char*>(F->resolveMeta.ptr), &rimage, &offViews, &rblocks));
+                              static_cast<char*>(F->resolveMeta.ptr), &rimage, &offViews, &rblocks, true));
     }
     std::vector<ClearView> cv;
     uint32_t cblocks = 0;

@@ -339,6 +339,7 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
                       const DrawExtras& extras = DrawExtras{});
 // The resolve of numViews targets over instance records and prefix already in
 // device memory (a draw's metadata); uploads at most the per-view records.
+// The colour buffers count as cleared: every pixel is written, none is read.
 crx_status resolve_views_device(crx_context* ctx, const InstanceRec* instDev, const uint64_t* prefixDev,
                                 uint32_t numInstances, const crx_render_target* targets, uint32_t numViews,
                                 crx_display_attribute attribute, hipStream_t stream);
@@ -359,7 +360,7 @@ void view_targets(const crx_view* views, uint32_t numViews, uint64_t* const* fra
 size_t resolve_image_layout(uint32_t numInstances, uint32_t numViews, size_t* offPrefix, size_t* offViews);
 crx_status resolve_image(const crx_cmesh* instances, uint32_t numInstances, const uint64_t* prefix,
                          const crx_render_target* targets, uint32_t numViews, crx_display_attribute attribute,
-                         char* dev, std::vector<char>* image, size_t* offViews, uint32_t* blocks);
+                         char* dev, std::vector<char>* image, size_t* offViews, uint32_t* blocks, bool fresh);
 crx_status clear_records(uint64_t* const* buffers, const uint32_t* numPixels, uint32_t n, std::vector<ClearView>* cv,
                          uint32_t* blocks);
 

@@ -90,6 +90,52 @@ __device__ __forceinline__ float rcp_rn(float b) {
     return r;
 }
 
+// RN(sqrt(x)) for normal x in [kSqrtLo, kSqrtHi): v_rsq_f32 and the coupled
+// square root / half reciprocal iteration in fused multiply-adds with a final
+// residual correction (Markstein; Muller et al., Handbook of Floating-Point
+// Arithmetic, on FMA-based square root).  crx_check_division compares it with
+// the IEEE square root for every float of the range.
+constexpr float kSqrtLo = 0x1p-96f, kSqrtHi = 0x1p96f;
+
+__device__ __forceinline__ float sqrt_refined(float x) {
+    const float r = __builtin_amdgcn_rsqf(x);
+    float g = x * r, h = 0.5f * r;
+    const float e = __builtin_fmaf(-h, g, 0.5f);
+    g = __builtin_fmaf(g, e, g);
+    h = __builtin_fmaf(h, e, h);
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+}
+
+// normalize3 with the short sequences: the scale is RN(1 / RN(sqrt(v.v))) either way.
+__device__ __forceinline__ f3 normalize3_rn(f3 v) {
+    const float x = dot3(v, v);
+    float s;
+    if (__ballot(!(x >= kSqrtLo && x < kSqrtHi)) == 0ull) s = rcp_refined(sqrt_refined(x));
+    else s = 1.0f / sqrtf(x);
+    return scale3(v, s);
+}
+
+// RN(a / b) for lanes whose operands may be anything: the short sequence when
+// every active lane is in its range, else the IEEE division.
+__device__ __forceinline__ float div_rn(float a, float b) {
+    const float ma = fabsf(a), mb = fabsf(b);
+    if (__ballot(!(ma >= kDivLo && ma <= kDivHi && mb >= kDivLo && mb <= kDivHi)) == 0ull)
+        return div_fast(a, b, rcp_refined(b));
+    return a / b;
+}
+
+// f2u8 of any float: v_cvt_u32_f32 truncates, takes NaN and negatives to 0 and
+// saturates (a C++ cast of such values is undefined).
+__device__ __forceinline__ uint32_t f2u8_dev(float x) {
+    uint32_t r;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return min(r, 255u);
+}
+
+// fmodf(x, m) for 0 < m, -m < x < 2m or NaN x: x itself below m, else x - m,
+// which is exact (Sterbenz).
+__device__ __forceinline__ float fmod_once(float x, float m) { return x >= m ? x - m : x; }
+
 // Orders LDS traffic between the lanes of one wave (no hardware barrier: the
 // waves of a workgroup run independent loops here).
 __device__ __forceinline__ void wave_sync() {
@@ -2604,7 +2650,7 @@ __global__ __launch_bounds__(256) void k_stage3(RasterParams P) {
                 const int py = f2i(fy0 + (float)fragY);
                 if (py >= V.H) break;
                 const float v = 2.0f * ((float)py + 0.5f) / V.Hf - 1.0f;
-                const f3 dir = normalize3(f3{rx, V.fI * v, -1.0f});
+                const f3 dir = normalize3_rn(f3{rx, V.fI * v, -1.0f});
                 const float t = intersect_mt(T, dir);
                 if (t == __builtin_inff()) continue;
                 // depth = dot(t*dir, (0,0,-1)) (:734)
@@ -2621,7 +2667,7 @@ namespace {
 __device__ __forceinline__ float intersect_plane(f3 origin, f3 dir, f3 normal, float constant) {
     const float denominator = dot3(normal, dir);
     if (denominator == 0.0f) return __builtin_inff();
-    const float t = -(dot3(origin, normal) + constant) / denominator;
+    const float t = div_rn(-(dot3(origin, normal) + constant), denominator);
     return (t >= 0.0f) ? t : __builtin_inff();
 }
 
@@ -2629,10 +2675,11 @@ __device__ __forceinline__ float intersect_plane(f3 origin, f3 dir, f3 normal, f
 // (resolve.cu:736-1035).  `mesh` is a register copy of the instance record.
 // computeRayDir (resolve.cu:662-676) through the screen point (px, py).
 __device__ __forceinline__ f3 resolve_ray(const ResolveParams& R, const f3& origin, float px, float py) {
-    const float u = 2.0f * px / R.Wf - 1.0f;
-    const float v = 2.0f * py / R.Hf - 1.0f;
-    const f3 rview = normalize3(f3{R.p00I * u, R.p11I * v, -1.0f});
-    return normalize3(sub3(xform_point(R.viewI, rview), origin));
+    // px, py are at least 0.5 and the size at most 2^31: div_fast's range
+    const float u = div_fast(2.0f * px, R.Wf, R.WI) - 1.0f;
+    const float v = div_fast(2.0f * py, R.Hf, R.HI) - 1.0f;
+    const f3 rview = normalize3_rn(f3{R.p00I * u, R.p11I * v, -1.0f});
+    return normalize3_rn(sub3(xform_point(R.viewI, rview), origin));
 }
 
 // sampleColor_linear (resolve.cu:148-195): the four texels around the sample
@@ -2645,8 +2692,9 @@ __device__ __forceinline__ uint32_t sample_linear(const uint32_t* data, int widt
     const auto tex = kglobal(data);
     const int last = width * height - 1;
     auto texel = [&](float fx, float fy) -> uint32_t {
-        const int tx = f2i(fmodf(fx, fw));
-        const int ty = f2i(fmodf(fy, fh));
+        // -0.5 <= fx <= fw + 0.5 (or NaN), and fw >= 1
+        const int tx = f2i(fmod_once(fx, fw));
+        const int ty = f2i(fmod_once(fy, fh));
         int id = tx + ty * width;
         id = id < 0 ? 0 : (id > last ? last : id);
         return tex[id];
@@ -2655,8 +2703,9 @@ __device__ __forceinline__ uint32_t sample_linear(const uint32_t* data, int widt
     const uint32_t t01 = texel(ftx - 0.5f, fty + 0.5f);
     const uint32_t t10 = texel(ftx + 0.5f, fty - 0.5f);
     const uint32_t t11 = texel(ftx + 0.5f, fty + 0.5f);
-    const float wx = fmodf(ftx + 0.5f, 1.0f);
-    const float wy = fmodf(fty + 0.5f, 1.0f);
+    // fmodf(x, 1) of x >= 0
+    const float wx = (ftx + 0.5f) - floorf(ftx + 0.5f);
+    const float wy = (fty + 0.5f) - floorf(fty + 0.5f);
     const float w00 = (1.0f - wx) * (1.0f - wy), w10 = wx * (1.0f - wy), w01 = (1.0f - wx) * wy, w11 = wx * wy;
     uint32_t rgb = 0u;
     #pragma unroll
@@ -2664,7 +2713,7 @@ __device__ __forceinline__ uint32_t sample_linear(const uint32_t* data, int widt
         const float c = ((w00 * (float)((t00 >> (8 * k)) & 0xffu) + w10 * (float)((t10 >> (8 * k)) & 0xffu)) +
                          w01 * (float)((t01 >> (8 * k)) & 0xffu)) +
                         w11 * (float)((t11 >> (8 * k)) & 0xffu);
-        rgb |= f2u8(c) << (8 * k);
+        rgb |= f2u8_dev(c) << (8 * k);
     }
     return 0xff000000u | rgb;
 }
@@ -2704,7 +2753,7 @@ __device__ __forceinline__ uint32_t shade_pixel(const ResolveParams& R, const In
         const f3 v0 = sub3(bw, aw);
         const f3 v1 = sub3(cw, aw);
         // resolve.cu:790-801
-        const f3 normal = normalize3(cross3(v0, v1));
+        const f3 normal = normalize3_rn(cross3(v0, v1));
         const float d = dot3(aw, normal);
         const float t = intersect_plane(origin, rayDir, normal, -d);
         // resolve.cu:805-834
@@ -2712,7 +2761,7 @@ __device__ __forceinline__ uint32_t shade_pixel(const ResolveParams& R, const In
         const float d01 = dot3(v0, v1);
         const float d11 = dot3(v1, v1);
         const float denom = d00 * d11 - d01 * d01;
-        const float denomI = 1.0f / denom;
+        const float denomI = rcp_rn(denom);
         // barycentric (s, t) of the ray's hit on the triangle's plane
         auto stv = [&](float th, const f3& rd, float& s_, float& t_) {
             const f3 p = add3(origin, f3{th * rd.x, th * rd.y, th * rd.z});
@@ -2818,8 +2867,10 @@ __device__ __forceinline__ uint32_t shade_pixel(const ResolveParams& R, const In
             float uy = (ua[1] * w + ub[1] * stx) + uc[1] * sty;
             ux = ux - floorf(ux);
             uy = uy - floorf(uy);
-            const uint32_t r = f2u8(fmodf(ux - floorf(ux), 1.0f) * 256.0f);
-            const uint32_t g = f2u8(fmodf(uy - floorf(uy), 1.0f) * 256.0f);
+            // fmodf(x, 1) of x in [0, 1] (or NaN)
+            const float fx = ux - floorf(ux), fy = uy - floorf(uy);
+            const uint32_t r = f2u8_dev((fx - floorf(fx)) * 256.0f);
+            const uint32_t g = f2u8_dev((fy - floorf(fy)) * 256.0f);
             color = (color & 0xff000000u) | r | (g << 8);
         } else if (attr == 3) {                // NORMAL
             f3 N;
@@ -2827,17 +2878,17 @@ __device__ __forceinline__ uint32_t shade_pixel(const ResolveParams& R, const In
                 const f3 n0 = xform(mesh.world, load_pos(mesh.normals, i0), 0.0f);
                 const f3 n1 = xform(mesh.world, load_pos(mesh.normals, i1), 0.0f);
                 const f3 n2 = xform(mesh.world, load_pos(mesh.normals, i2), 0.0f);
-                N = normalize3(add3(add3(scale3(n0, w), scale3(n1, stx)), scale3(n2, sty)));
+                N = normalize3_rn(add3(add3(scale3(n0, w), scale3(n1, stx)), scale3(n2, sty)));
             } else {
-                N = normalize3(cross3(v0, v1));
+                N = normalize3_rn(cross3(v0, v1));
             }
-            const uint32_t r = f2u8(clampf(N.x * 255.0f, 0.0f, 255.0f));
-            const uint32_t g = f2u8(clampf(N.y * 255.0f, 0.0f, 255.0f));
-            const uint32_t b = f2u8(clampf(N.z * 255.0f, 0.0f, 255.0f));
+            const uint32_t r = f2u8_dev(N.x * 255.0f);
+            const uint32_t g = f2u8_dev(N.y * 255.0f);
+            const uint32_t b = f2u8_dev(N.z * 255.0f);
             color = (color & 0xff000000u) | r | (g << 8) | (b << 16);
         } else if (attr == 4 && mesh.colors) { // VERTEX_COLORS (resolve.cu:952-973)
             const auto colors = kglobal(mesh.colors);
-        const uint32_t Ca = colors[i0], Cb = colors[i1], Cc = colors[i2];
+            const uint32_t Ca = colors[i0], Cb = colors[i1], Cc = colors[i2];
             uint32_t rgb = 0;
             #pragma unroll
             for (int k = 0; k < 3; k++) {
@@ -2845,7 +2896,7 @@ __device__ __forceinline__ uint32_t shade_pixel(const ResolveParams& R, const In
                 const float cb = (float)((Cb >> (8 * k)) & 0xffu);
                 const float cc = (float)((Cc >> (8 * k)) & 0xffu);
                 const float ch = (ca * w + cb * stx) + cc * sty;
-                rgb |= f2u8(clampf(ch, 0.0f, 255.0f)) << (8 * k);
+                rgb |= f2u8_dev(ch) << (8 * k);   // clamps to [0, 255]
             }
             color = (Ca & 0xff000000u) | rgb;
         } else {
@@ -2862,11 +2913,14 @@ __device__ __forceinline__ void resolve_pixel(const ResolveParams& R, int x, int
     const uint32_t pixelID = (uint32_t)x + (uint32_t)R.W * (uint32_t)y;
 
     const uint64_t pixel = kglobal(R.fb)[pixelID];
-    const uint64_t pixel_cb = kglobal((const uint64_t*)R.cb)[pixelID];
     const float depth = unpack_depth(pixel);
     const uint64_t total = pixel & 0xFFFFFFFFFull;
-    const float depth_cb = __builtin_bit_cast(float, (uint32_t)(pixel_cb >> 32));
-    if (depth_cb < depth) return;
+    // a fresh colour buffer holds the clear pixel, whose depth (a NaN) stops nothing
+    if (!R.fresh) {
+        const uint64_t pixel_cb = kglobal((const uint64_t*)R.cb)[pixelID];
+        const float depth_cb = __builtin_bit_cast(float, (uint32_t)(pixel_cb >> 32));
+        if (depth_cb < depth) return;
+    }
 
     uint32_t color = 0;
     if (!__builtin_isinf(depth) && R.numInstances > 0) {
@@ -2874,7 +2928,7 @@ __device__ __forceinline__ void resolve_pixel(const ResolveParams& R, int x, int
         const uint32_t n = R.numInstances;
         const auto prefix = kglobal(R.prefix);
         int left = 0, right = (int)(n - 1u), found = 0;
-        while (left <= right) {
+        while (n > 1u && left <= right) {   // (a lone instance is always the one found)
             const int mid = left + (right - left) / 2;
             const int64_t before = (int64_t)prefix[mid];
             const int64_t after = ((uint32_t)mid == n - 1u) ? 0xffffffffffll : (int64_t)prefix[mid + 1];
@@ -2980,7 +3034,8 @@ __global__ __launch_bounds__(256) void k_copy(u32x4* __restrict__ dst, const u32
 
 // Check of rcp_refined / div_fast against the IEEE division: lanes sweep all
 // floats b with kRcpLo <= |b| < kRcpHi (biased exponents 2..251, both signs)
-// and count b with rcp_refined(b) != 1/b (out[0]); then `pairs` hashed
+// and count b with rcp_refined(b) != 1/b, or, in [kSqrtLo, kSqrtHi),
+// sqrt_refined(b) != sqrt(b) (out[0]); then `pairs` hashed
 // operand pairs (a, b) with exponents in [-60, 63] and any mantissa and sign
 // count div_fast(a, b, rcp_refined(b)) != a/b (out[1]), and as many pairs
 // with |a| below kDivLo (zero and subnormals included) count
@@ -2997,6 +3052,8 @@ __global__ __launch_bounds__(256) void k_check_division(uint64_t pairs, unsigned
         const float r = rcp_refined(b);
         const float q = 1.0f / b;
         bad += __builtin_bit_cast(uint32_t, r) != __builtin_bit_cast(uint32_t, q) ? 1u : 0u;
+        if (b >= kSqrtLo && b < kSqrtHi)
+            bad += __builtin_bit_cast(uint32_t, sqrt_refined(b)) != __builtin_bit_cast(uint32_t, sqrtf(b)) ? 1u : 0u;
     }
     if (bad) atomicAdd(out, (unsigned long long)bad);
     bad = 0u;

@@ -487,10 +487,6 @@ crx_status draw_group(crx_server* s, crx_server::Lane& lane, const std::vector<R
         t.aspect = (float)cv.width / (float)cv.height;
         bufs.push_back(t.framebuffer);
         px.push_back((uint32_t)pixels);
-        if (t.colorbuffer) {
-            bufs.push_back(t.colorbuffer);
-            px.push_back((uint32_t)pixels);
-        }
     }
     // view-major transforms and per-view node culls of the nodes `ids`
     std::vector<crx_mat4> xf;
@@ -555,6 +551,12 @@ crx_status draw_group(crx_server* s, crx_server::Lane& lane, const std::vector<R
     std::vector<std::vector<uint32_t>> groups;
     for (size_t g0 = 0; g0 < need.size(); g0 += group)
         groups.emplace_back(need.begin() + g0, need.begin() + std::min(need.size(), g0 + group));
+    // (the resolve in passes reads the colour buffers: they are cleared too)
+    for (uint32_t v = 0; v < V; v++) {
+        if (!targets[v].colorbuffer) continue;
+        bufs.push_back(targets[v].colorbuffer);
+        px.push_back(px[v]);
+    }
     CRX_TRY(clear_buffers(lane.ctx, bufs.data(), px.data(), (uint32_t)bufs.size(), lane.stream));
     const auto pass = [&](const std::vector<uint32_t>& ids, bool resolvePass) -> crx_status {
         uint32_t up = 0;
