@@ -221,17 +221,6 @@ __device__ __forceinline__ uint32_t item_cull_order(const RasterParams& P, uint3
 //    screen transform, with slack); only triangles that are culled for sure
 //    leave early, all others take the exact path.
 //
-// stage1_core takes each vertex's depth d = -view.z and, with PRE, its view
-// y row (VQ), from a caller that computed them once for vertices shared
-// between triangles: the same operations, so the same bits.
-struct VQ {
-    float d, y;
-};
-
-__device__ __forceinline__ VQ vertex_q(const float* m, f3 p) {
-    return VQ{-xform_row(m, 2, p), xform_row(m, 1, p)};
-}
-
 //
 // DEFER: the function neither draws nor queues.  It tells what is to be done
 // with the triangle, for a caller that does it for its lanes together
@@ -245,30 +234,26 @@ struct RasterTri {
     bool fast;                           // depths in the range of the short reciprocal
 };
 
-template <bool PRE, bool DEFER = false, bool INSIDE = false>
+template <bool DEFER>
 __device__ __forceinline__ S1Result stage1_core(const RasterParams& P, const ViewParams& V, const float* __restrict__ m,
-                                            bool flip, f3 A, f3 B, f3 C, const VQ& qa, const VQ& qb, const VQ& qc,
-                                            uint64_t id, uint64_t queueEntry, uint32_t cullOrder,
-                                            RasterTri* rt = nullptr, bool inside = false) {
-    const float da = qa.d, db = qb.d, dc = qc.d;
-    // inside (wave-uniform, known with INSIDE): every vertex lies in front of
-    // the camera and between the side planes by a margin (view_inside), so
-    // the tests against them are decided
-    inside = INSIDE && inside;
+                                                bool flip, f3 A, f3 B, f3 C, uint64_t id, uint64_t queueEntry,
+                                                uint32_t cullOrder, RasterTri* rt = nullptr) {
+    // depth first: ndc.z = depth = -view.z
+    const float da = -xform_row(m, 2, A), db = -xform_row(m, 2, B), dc = -xform_row(m, 2, C);
     // all vertices behind the camera (:119)
-    if (!inside && da <= 0.0f && db <= 0.0f && dc <= 0.0f) return S1_NONE;
-    bool nontrivial = !inside && (da <= 0.0f || db <= 0.0f || dc <= 0.0f);
-    const bool safeDepth = inside || (da >= 0x1p-102f && db >= 0x1p-102f && dc >= 0x1p-102f);
+    if (da <= 0.0f && db <= 0.0f && dc <= 0.0f) return S1_NONE;
+    bool nontrivial = da <= 0.0f || db <= 0.0f || dc <= 0.0f;
+    const bool safeDepth = da >= 0x1p-102f && db >= 0x1p-102f && dc >= 0x1p-102f;
     const float fa = V.fa, f = V.f;
 
     // frustum culling (:113-118), only when every depth is positive; the axis
     // the view culls most is tested before the other coordinate is computed
     const bool frustumFirst = cullOrder != 0;
-    float vya = qa.y, vyb = qb.y, vyc = qc.y, vxa = 0.0f, vxb = 0.0f, vxc = 0.0f;
-    bool haveX = false, haveY = PRE;
-    if (frustumFirst && !inside && !nontrivial && safeDepth) {
+    float vya = 0.0f, vyb = 0.0f, vyc = 0.0f, vxa = 0.0f, vxb = 0.0f, vxc = 0.0f;
+    bool haveX = false, haveY = false;
+    if (frustumFirst && !nontrivial && safeDepth) {
         if (cullOrder == 1) {
-            if (!PRE) { vya = xform_row(m, 1, A); vyb = xform_row(m, 1, B); vyc = xform_row(m, 1, C); }
+            vya = xform_row(m, 1, A); vyb = xform_row(m, 1, B); vyc = xform_row(m, 1, C);
             haveY = true;
             if (frustum_culled_axis(f * vya, f * vyb, f * vyc, da, db, dc)) return S1_NONE;
             vxa = xform_row(m, 0, A); vxb = xform_row(m, 0, B); vxc = xform_row(m, 0, C);
@@ -278,7 +263,7 @@ __device__ __forceinline__ S1Result stage1_core(const RasterParams& P, const Vie
             vxa = xform_row(m, 0, A); vxb = xform_row(m, 0, B); vxc = xform_row(m, 0, C);
             haveX = true;
             if (frustum_culled_axis(fa * vxa, fa * vxb, fa * vxc, da, db, dc)) return S1_NONE;
-            if (!PRE) { vya = xform_row(m, 1, A); vyb = xform_row(m, 1, B); vyc = xform_row(m, 1, C); }
+            vya = xform_row(m, 1, A); vyb = xform_row(m, 1, B); vyc = xform_row(m, 1, C);
             haveY = true;
             if (frustum_culled_axis(f * vya, f * vyb, f * vyc, da, db, dc)) return S1_NONE;
         }
@@ -297,7 +282,7 @@ __device__ __forceinline__ S1Result stage1_core(const RasterParams& P, const Vie
         if (flip) res = -res;
         if (res >= 0.0f) return S1_NONE;
     }
-    if (!frustumFirst && !inside && !nontrivial) {
+    if (!frustumFirst && !nontrivial) {
         if (safeDepth) {
             if (frustum_culled_axis(pxa, pxb, pxc, da, db, dc) || frustum_culled_axis(pya, pyb, pyc, da, db, dc))
                 return S1_NONE;
@@ -449,12 +434,7 @@ __device__ __forceinline__ void stage1_triangle(const RasterParams& P, const Vie
                                                 const float* __restrict__ m,
                                                 bool flip, f3 A, f3 B, f3 C,
                                                 uint64_t id, uint64_t queueEntry, uint32_t cullOrder) {
-    // depth first: ndc.z = depth = -view.z
-    VQ qa{}, qb{}, qc{};
-    qa.d = -xform_row(m, 2, A);
-    qb.d = -xform_row(m, 2, B);
-    qc.d = -xform_row(m, 2, C);
-    stage1_core<false>(P, V, m, flip, A, B, C, qa, qb, qc, id, queueEntry, cullOrder);
+    stage1_core<false>(P, V, m, flip, A, B, C, id, queueEntry, cullOrder);
 }
 
 }  // namespace
@@ -1198,13 +1178,14 @@ __device__ __forceinline__ bool view_may_see(const ViewCull& c, const WaveBox& B
 
 // True only when every vertex in the box lies in front of the camera and
 // inside the side planes, for the per-triangle code as well: its computed
-// depths are positive (at least 2^-90) and no quotient's magnitude exceeds 1.
+// depths are positive (at least 2^-90, and at most 2^100, so that v_rcp_f32
+// serves the filter of k_stage1_pairs) and no quotient's magnitude exceeds 1.
 // The margins are view_may_see's, on the other side of the planes.
 __device__ __forceinline__ bool view_inside(const ViewCull& c, const WaveBox& B) {
     const float mz = (c.slopeZ * B.M + c.cnstZ) * 0x1p-16f + 0x1p-90f;
     const float mx = (c.slopeX * B.M + c.cnstX) * 0x1p-16f + 0x1p-90f;
     const float my = (c.slopeY * B.M + c.cnstY) * 0x1p-16f + 0x1p-90f;
-    return box_max(c.z, B) < -mz && box_max(c.px, B) < -mx && box_max(c.nx, B) < -mx && box_max(c.py, B) < -my &&
+    return box_max(c.z, B) < -mz && box_min(c.z, B) > -0x1p99f && mz < 0x1p99f && box_max(c.px, B) < -mx && box_max(c.nx, B) < -mx && box_max(c.py, B) < -my &&
            box_max(c.ny, B) < -my;
 }
 
@@ -1571,12 +1552,7 @@ __global__ __launch_bounds__(256) void k_stage1_coarse(RasterParams P) {
             S1Result todo = S1_NONE;
             const uint64_t entry = ((uint64_t)inst << 32) | (uint64_t)tri;
             if (tri < it.numTriangles) {
-                VQ qa{}, qb{}, qc{};
-                qa.d = -xform_row(m, 2, A);
-                qb.d = -xform_row(m, 2, B);
-                qc.d = -xform_row(m, 2, C);
-                todo = stage1_core<false, true>(P, V0, m, T->flip != 0u, A, B, C, qa, qb, qc, id, entry, cullOrder,
-                                                &rt);
+                todo = stage1_core<true>(P, V0, m, T->flip != 0u, A, B, C, id, entry, cullOrder, &rt);
             }
             // the stage-2 entries of the workgroup, appended with one atomic
             // (each returning atomic on the one counter takes 6 ns)
@@ -1910,7 +1886,8 @@ __device__ __forceinline__ uint32_t pair_vertices(const S1Item& it, uint32_t bas
 // s1_sweep: while batch i is drawn, the gathers of batch i+1 and the index
 // loads of batch i+2 are in flight.  Units (strip, group of rows) are dealt
 // to the workgroups by P.order as s1_range deals batches; a workgroup walks
-// its unit's rows in turn.  body(it, base, end, S, pattern) draws one batch.
+// its unit's rows in turn.  body(it, base, end, S, pattern, inside, last)
+// draws one batch; `last` marks the last one of a pass over an item.
 template <bool PU16, bool LISTED, typename Body>
 __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* words, Body&& body) {
     const uint32_t numUnits = P.batchCount ? *kconst(P.batchCount) : P.numBatches;
@@ -1970,7 +1947,7 @@ __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* 
                     S[5] = pu16_vertex_decode(it, S[5]);
                 }
             }
-            body(it, base0, end0, S, pat, inside != 0u);
+            body(it, base0, end0, S, pat, inside != 0u, !more1);
             if (!more1) break;
             inside = b1.inside;
             base0 = base1;
@@ -1988,8 +1965,99 @@ __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* 
     }
 }
 
+namespace {
+
+// Screen position of a vertex within a small margin of the exact one, for
+// the filter of k_stage1_pairs: the exact view rows, and the quotients as
+// products with v_rcp_f32.  With |ndc| <= 2 the quotient is within 2^-21 of
+// the IEEE one and the screen coordinate, with the roundings of both screen
+// transforms, within 2^-20.7 * size; the filter's margin is 2^-19 * max(W, H).
+struct FilterView {
+    float gx, gy, cx, cy;    // half a size times the focal factor, and the screen centre
+    float W, H, margin;
+};
+
+__device__ __forceinline__ FilterView filter_view(const ViewParams& V) {
+    const float hx = 0.5f * V.Wf, hy = 0.5f * V.Hf;
+    return FilterView{V.fa * hx, V.f * hy, hx - 0.5f, hy - 0.5f, V.Wf, V.Hf, fmaxf(V.Wf, V.Hf) * 0x1p-19f};
+}
+
+struct FV {
+    float x, y, d;
+};
+
+__device__ __forceinline__ FV filter_vertex(const FilterView& F, const float* m, f3 p) {
+    FV v;
+    v.d = -xform_row(m, 2, p);
+    const float r = __builtin_amdgcn_rcpf(v.d);
+    v.x = __builtin_fmaf(xform_row(m, 0, p), F.gx * r, F.cx);
+    v.y = __builtin_fmaf(xform_row(m, 1, p), F.gy * r, F.cy);
+    return v;
+}
+
+// True only when the exact code (stage1_core) neither draws nor queues the
+// triangle.  All behind the camera: culled.  Otherwise, with every depth in
+// [2^-100, 2^100], when its box lies off one side by a sample or more (all
+// quotients beyond 1 in magnitude by more than the margin: the frustum test
+// culls it), or strictly between two neighbouring sample rows or columns k - 1
+// and k.  For 0 < k < size the tiny-triangle test culls that; for k = size
+// too, as the clamp brings the box's upper end to size - 1 only; for k = 0
+// the clamped box holds no sample (size_x or size_y is 0); beyond those the
+// frustum test has it.  Coordinates further off have larger errors, but
+// which of the cases they fall in does not depend on those.  A NaN or
+// infinite coordinate is NaN or infinite in both.
+__device__ __forceinline__ bool filter_culls(const FilterView& F, bool inside, const FV& a, const FV& b, const FV& c) {
+    const float lox = fminf(a.x, fminf(b.x, c.x)), hix = fmaxf(a.x, fmaxf(b.x, c.x));
+    const float loy = fminf(a.y, fminf(b.y, c.y)), hiy = fmaxf(a.y, fmaxf(b.y, c.y));
+    const bool tiny = (hix + F.margin < ceilf(lox - F.margin)) | (hiy + F.margin < ceilf(loy - F.margin));
+    if (inside) return tiny;   // wave-uniform: the depths are positive and no side is crossed
+    const float dmin = fminf(a.d, fminf(b.d, c.d)), dmax = fmaxf(a.d, fmaxf(b.d, c.d));
+    const bool safe = (dmin >= 0x1p-100f) & (dmax <= 0x1p100f) & (a.d == a.d) & (b.d == b.d) & (c.d == c.d);
+    const bool behind = (a.d <= 0.0f) & (b.d <= 0.0f) & (c.d <= 0.0f);
+    return behind | (safe & (tiny | (lox > F.W) | (hix < -1.0f) | (loy > F.H) | (hiy < -1.0f)));
+}
+
+// Rank of the lane among the lanes of a mask.
+__device__ __forceinline__ uint32_t mask_rank(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// The triangles that the filter left, per wave: fewer than 64 from earlier
+// batches and up to 128 of this one.
+struct LeftTris {
+    float p[9][3 * kWave];
+    uint32_t tri[3 * kWave];
+
+    __device__ __forceinline__ void put(uint32_t at, uint32_t t, const f3& a, const f3& b, const f3& c) {
+        p[0][at] = a.x; p[1][at] = a.y; p[2][at] = a.z;
+        p[3][at] = b.x; p[4][at] = b.y; p[5][at] = b.z;
+        p[6][at] = c.x; p[7][at] = c.y; p[8][at] = c.z;
+        tri[at] = t;
+    }
+    __device__ __forceinline__ uint32_t get(uint32_t at, f3& a, f3& b, f3& c) const {
+        a = f3{p[0][at], p[1][at], p[2][at]};
+        b = f3{p[3][at], p[4][at], p[5][at]};
+        c = f3{p[6][at], p[7][at], p[8][at]};
+        return tri[at];
+    }
+};
+
+}  // namespace
+
 // Stage 1 over pairs of consecutive triangles for draws of one view whose
 // items are drawn over few instances (the others take k_stage1).
+//
+// Bound by VALU issue before it is by memory: the exact code takes about 280
+// instructions per 64 triangles, and most of a large mesh's triangles hold no
+// sample (2.4% of a 25 M-triangle terrain seen whole at 720p draw one, so that
+// their pixels ran with 4 of 64 lanes).  So each batch passes a filter first,
+// on the vertices the pair shares (filter_vertex: 18 instructions for the exact
+// view rows and 8 for an approximate projection), and only what it leaves is
+// gathered in LDS and drawn 64 at a time by the exact code.  The positions are
+// kept with them: gathered again from memory they made the kernel fetch 600
+// MB in place of 520 and wait (143 us against 134).
+// Stage 1 of that terrain 195 -> 130 us (VALU instructions 112 M -> 50 M, 4.0
+// TB/s fetched), of the 400 M-triangle one's 1.5% in view 79 -> 62.
 template <int BLOCK, bool PU16, bool LISTED>
 __global__ __launch_bounds__(BLOCK) void k_stage1_pairs(RasterParams P) {
     const ViewParams V0 = kconst(P.views)[0];
@@ -1999,9 +2067,14 @@ __global__ __launch_bounds__(BLOCK) void k_stage1_pairs(RasterParams P) {
         __shared__ __align__(16) uint32_t pairWords[BLOCK / kWave][kPairPu16Words];
         words = pairWords[threadIdx.x / kWave];
     }
-    s1_pairs_sweep<PU16, LISTED>(P, words, [&](const S1Item& it, uint32_t base, uint32_t end, const f3 (&S)[6], uint32_t pat, bool inside)
-                          __attribute__((always_inline)) {
-        const uint32_t ta = base + 2u * (threadIdx.x & (kWave - 1)), tb = ta + 1u;
+    __shared__ LeftTris leftTris[BLOCK / kWave];
+    LeftTris& left = leftTris[threadIdx.x / kWave];
+    const FilterView F = filter_view(V0);
+    uint32_t queued = 0;
+    s1_pairs_sweep<PU16, LISTED>(P, words, [&](const S1Item& it, uint32_t base, uint32_t end, const f3 (&S)[6],
+                                               uint32_t pat, bool inside, bool last) __attribute__((always_inline)) {
+        const uint32_t lane = threadIdx.x & (kWave - 1);
+        const uint32_t ta = base + 2u * lane, tb = ta + 1u;
         for (uint32_t j = 0; j < it.instCount; j++) {
             const uint32_t inst = it.instOffset + j;
             const auto T = transforms + inst;
@@ -2009,22 +2082,42 @@ __global__ __launch_bounds__(BLOCK) void k_stage1_pairs(RasterParams P) {
             #pragma unroll
             for (int e = 0; e < 16; e++) m[e] = T->m[e];
             const bool flip = T->flip != 0u;
-            const uint32_t cullOrder = item_cull_order(P, it.instCount);
-            const uint64_t off = it.cumm + (uint64_t)(j * it.numTriangles);
-            const uint64_t hi = (uint64_t)inst << 32;
-            if (pat != kPairNone) {
-                // the four distinct vertices' quantities, once
-                const VQ q0 = vertex_q(m, S[0]), q1 = vertex_q(m, S[1]), q2 = vertex_q(m, S[2]), q3 = vertex_q(m, S[3]);
-                if (ta < end) stage1_core<true, false, LISTED>(P, V0, m, flip, S[0], S[1], S[2], q0, q1, q2, off + ta, hi | ta, cullOrder, nullptr, inside);
-                // B = (A.a, A.c, n) or (A.a, n, A.b): a wave-uniform choice
-                if (pat == kPairGrid) {
-                    if (tb < end) stage1_core<true, false, LISTED>(P, V0, m, flip, S[0], S[2], S[3], q0, q2, q3, off + tb, hi | tb, cullOrder, nullptr, inside);
-                } else {
-                    if (tb < end) stage1_core<true, false, LISTED>(P, V0, m, flip, S[0], S[3], S[1], q0, q3, q1, off + tb, hi | tb, cullOrder, nullptr, inside);
-                }
-            } else {
-                if (ta < end) stage1_triangle(P, V0, m, flip, S[0], S[1], S[2], off + ta, hi | ta, cullOrder);
-                if (tb < end) stage1_triangle(P, V0, m, flip, S[3], S[4], S[5], off + tb, hi | tb, cullOrder);
+            const FV v0 = filter_vertex(F, m, S[0]), v1 = filter_vertex(F, m, S[1]), v2 = filter_vertex(F, m, S[2]),
+                     v3 = filter_vertex(F, m, S[3]);
+            const bool keepA = ta < end && !filter_culls(F, LISTED && inside, v0, v1, v2);
+            FV b0 = v0, b1 = v3, b2 = v1;                     // kPairFan: (A.a, n, A.b)
+            if (pat == kPairGrid) {                           // (A.a, A.c, n)
+                b1 = v2;
+                b2 = v3;
+            } else if (pat == kPairNone) {
+                b0 = v3;
+                b1 = filter_vertex(F, m, S[4]);
+                b2 = filter_vertex(F, m, S[5]);
+            }
+            const bool keepB = tb < end && !filter_culls(F, LISTED && inside, b0, b1, b2);
+            const uint64_t ma = __ballot(keepA), mb = __ballot(keepB);
+            if (keepA) left.put(queued + mask_rank(ma), ta, S[0], S[1], S[2]);
+            queued += (uint32_t)__popcll(ma);
+            if (keepB) {
+                const uint32_t at = queued + mask_rank(mb);
+                if (pat == kPairGrid) left.put(at, tb, S[0], S[2], S[3]);
+                else if (pat == kPairFan) left.put(at, tb, S[0], S[3], S[1]);
+                else left.put(at, tb, S[3], S[4], S[5]);
+            }
+            queued += (uint32_t)__popcll(mb);
+            // what is left of an instance, or of the pass over an item, is drawn at its end
+            const bool all = last || it.instCount > 1u;
+            while (queued >= kWave || (all && queued > 0u)) {
+                const uint32_t n = min(queued, (uint32_t)kWave);
+                queued -= n;
+                wave_sync();
+                f3 A, B, C;
+                const uint32_t t = left.get(queued + min(lane, n - 1u), A, B, C);
+                wave_sync();
+                const uint64_t id = it.cumm + (uint64_t)t + (uint64_t)(j * it.numTriangles);
+                if (lane < n)
+                    stage1_triangle(P, V0, m, flip, A, B, C, id, ((uint64_t)inst << 32) | t,
+                                    item_cull_order(P, it.instCount));
             }
         }
     });
