@@ -403,11 +403,27 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
     }
     // A draw of meshes whose units have boxes draws only the units the view
     // may see.  The boxes are those of the default walk.
-    if (bounds.boxes && !D.coarse && numViews == 1 && !manyInstances && D.block == 256 && tu.stage1_tris_per_lane == 0 &&
+    // Several views draw each unit once for every view that may see it.
+    const auto row_hint = [&](uint32_t k) {
+        return tu.stage1_layout != 2 ? 0u : bounds.rows ? bounds.rows[k] : row_hint_of(list[k].indices);
+    };
+    if (bounds.boxes && !D.coarse && !manyInstances && D.block == 256 && tu.stage1_tris_per_lane == 0 &&
         tu.stage1_layout == 2 && tu.stage1_strip_rows == kUnitRows && tu.stage1_strip_batches == 1) {
         uint64_t tris = 0;
         for (uint32_t k = 0; k < D.numItems; k++) tris += bounds.boxes[k] ? list[k].numTriangles : 0u;
         D.listed = bounds.always || tris >= kListMinTris;
+        if (D.listed && numViews > 1) {
+            uint64_t units = 0;
+            bool longRows = false;
+            for (uint32_t k = 0; k < D.numItems; k++) {
+                DrawItem it{};
+                it.numTriangles = list[k].numTriangles;
+                units += pair_layout(it, row_hint(k), tu.stage1_strip_rows, tu.stage1_strip_batches);
+                longRows = longRows || it.rowTris > kListMaxRowTris;
+            }
+            // (k_stage1_pairs' squares address eight rows of indices with 32 bits)
+            D.listed = units * numViews <= kListMaxEntries && !longRows;
+        }
         if (D.listed) D.runs = true;
     }
 
@@ -442,8 +458,7 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
         it.cf[0] = m.compressionFactor.x; it.cf[1] = m.compressionFactor.y; it.cf[2] = m.compressionFactor.z;
         it.amin[0] = m.aabb.min.x; it.amin[1] = m.aabb.min.y; it.amin[2] = m.aabb.min.z;
         it.numVertices = m.numVertices;
-        const uint32_t rowHint = (D.runs && tu.stage1_layout == 2) ? row_hint_of(m.indices) : 0u;
-        const uint64_t units = pair_layout(it, rowHint, tu.stage1_strip_rows, tu.stage1_strip_batches);
+        const uint64_t units = pair_layout(it, D.runs ? row_hint(k) : 0u, tu.stage1_strip_rows, tu.stage1_strip_batches);
         if (D.listed) it.bounds = bounds.boxes[k];
         D.batches += D.runs ? units : ((uint64_t)m.numTriangles + batchTris - 1) >> D.batchShift;
         D.tris += (uint64_t)m.numTriangles * (uint64_t)cnt;
@@ -545,7 +560,7 @@ hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& D, const RasterParam
         if (e != hipSuccess) return e;
     }
     record(ctx, T_S1, stream);
-    if (D.numViews == 1 && !viewsKernel && D.runs)
+    if (!viewsKernel && D.runs)
     {
         if (D.listed) e = launch_cull_units(P, stream);
         if (e == hipSuccess) e = launch_stage1_pairs(P, D.block, D.g1, D.pu16, D.listed, stream);
@@ -644,8 +659,8 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
         return finish();
     }
     CRX_TRY(ensure_queues(ctx, ctx->tuning.max_nontrivial, ctx->tuning.max_huge));
-    if (D.listed) CRX_TRY(ctx->unitList.reserve(D.batches * sizeof(uint32_t)));
-    P.units = static_cast<uint32_t*>(ctx->unitList.ptr);
+    if (D.listed) CRX_TRY(ctx->unitList.reserve(D.batches * D.numViews * sizeof(uint64_t)));
+    P.units = static_cast<uint64_t*>(ctx->unitList.ptr);
 
     uint32_t redraws = 0;
     for (;;) {
@@ -668,7 +683,7 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
             stats->num_nontrivial = nNt;
             stats->num_huge = nHuge;
             stats->redraws = redraws;
-            stats->stage1_kernel = D.numViews > 1 ? 1u : D.runs ? 2u : 0u;
+            stats->stage1_kernel = D.runs ? 2u : D.numViews > 1 ? 1u : 0u;
         }
         if (nNt <= ctx->ntCap && nHuge <= ctx->hugeCap) break;
         // Queue overflow: grow and draw again.  Every value the truncated pass

@@ -31,6 +31,12 @@ constexpr uint32_t kUnitRows = 8;
 // Triangles from which a mesh gets unit boxes and a draw uses them.
 constexpr uint64_t kListMinTris = 1u << 20;
 
+// Most entries (units times views) of a draw's unit list: 256 MB of list.
+constexpr uint64_t kListMaxEntries = 1u << 25;
+
+// Longest rows of a draw of several views from a unit list.
+constexpr uint32_t kListMaxRowTris = 1u << 24;
+
 // Stage-1 work unit.  Instanced draws: one unit per unique mesh that loops
 // over instCount consecutive instances.  Non-instanced draws: one unit per
 // instance (instCount == 1).
@@ -180,7 +186,7 @@ struct RasterParams {
     uint32_t numWaves2;      // waves in the stage-2 grid
     uint32_t numWaves3;      // waves in the stage-3 grid
     uint32_t splitShift;     // k_stage1_coarse: log2(lanes per triangle)
-    uint32_t* units;         // k_cull_units: the units left to draw ...
+    uint64_t* units;         // k_cull_units: the units left to draw, each with its view ...
     uint32_t* unitCount;     // ... and their number (CTR_UNITS)
     uint32_t* claims;        // k_stage1_pairs: the per-XCD unit counters (CTR_CLAIM of the counter block)
 };

@@ -106,7 +106,7 @@ crx_status frame_fill(crx_frame* F, bool write) {
     F->P.huge = static_cast<int4*>(F->huge.ptr);
     F->P.ntCap = F->ntCap;
     F->P.hugeCap = F->hugeCap;
-    F->P.units = static_cast<uint32_t*>(F->unitList.ptr);
+    F->P.units = static_cast<uint64_t*>(F->unitList.ptr);
     if (!rimage.empty()) std::memcpy(F->stageResolve, rimage.data(), rimage.size());
     if (!cv.empty()) std::memcpy(F->stageClear, cv.data(), F->clearBytes);
     return CRX_OK;
@@ -215,7 +215,7 @@ crx_status crx_frame_create(crx_context* ctx, crx_scene* scene, const crx_view* 
         F->hugeCap = ctx->tuning.max_huge;
         st = F->nontrivial.reserve((size_t)F->ntCap * sizeof(uint64_t));
         if (st == CRX_OK) st = F->huge.reserve((size_t)F->hugeCap * sizeof(int4));
-        if (st == CRX_OK && F->plan.listed) st = F->unitList.reserve(F->plan.batches * sizeof(uint32_t));
+        if (st == CRX_OK && F->plan.listed) st = F->unitList.reserve(F->plan.batches * numViews * sizeof(uint64_t));
     }
     hip(hipMalloc(&F->ctr, CTR_COUNT * sizeof(uint32_t)), "hipMalloc");
     hip(hipHostMalloc((void**)&F->ctrHost, CTR_COUNT * sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc");

@@ -133,11 +133,14 @@ struct DrawPlan {
     size_t offItems = 0, offInst = 0, offPrefix = 0, offViews = 0, offXf = 0, metaBytes = 0;
 };
 
-// Per draw item: the boxes of its mesh's units (crx_mesh::bounds), or null.
+// Per draw item: the boxes of its mesh's units (crx_mesh::bounds), or null,
+// and optionally the row length their layout was made for (else the one that
+// the index buffer's address is registered with).
 // always: list the units whatever the items' boxes (a recorded frame keeps
 // its layout when a mesh loses them).
 struct DrawBounds {
     const UnitBox* const* boxes = nullptr;
+    const uint32_t* rows = nullptr;
     bool always = false;
 };
 
@@ -324,6 +327,9 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
                      bool instUnchanged = false, bool prefix = false, const DrawBounds& bounds = DrawBounds{});
 // The pair layout of a mesh's units (DrawItem::rowTris ... unitCols); returns their number.
 uint64_t pair_layout(DrawItem& it, uint32_t rowHint, uint32_t stripRows, uint32_t stripBatches);
+
+// The row length of a mesh's index order (0: none found).
+uint32_t detect_row_triangles(const uint32_t* idx, uint64_t T);
 RasterParams plan_write(crx_context* ctx, const DrawPlan& plan, char* host, char* dev, bool writeInst = true);
 hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& plan, const RasterParams& P, bool viewsKernel,
                           hipStream_t stream, bool countersZeroed = false);

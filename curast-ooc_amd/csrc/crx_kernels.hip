@@ -1472,7 +1472,12 @@ __device__ __forceinline__ void raster_rows(const RasterTri& r, bool fast, uint6
 // scattered lanes/s against 206 G/s when 64 lanes hit 512 contiguous bytes).
 // So when enough lanes draw and their common box fits the wave's LDS tile,
 // the wave takes the minima there first; the minimum of minima is the same
-// value.
+// value.  The tile holds ~0 between calls (tile_clear at the kernel's start).
+__device__ __forceinline__ void tile_clear(uint64_t* tile) {
+    for (uint32_t k = threadIdx.x & (kWave - 1); k < kTilePixels; k += kWave) tile[k] = ~0ull;
+    wave_sync();
+}
+
 __device__ __forceinline__ void raster_wave(const ViewParams& V, uint64_t* tile, const RasterTri& r, bool has,
                                             uint64_t id, uint32_t slot, uint32_t step) {
     const uint64_t drawn = __ballot(has);
@@ -1487,19 +1492,21 @@ __device__ __forceinline__ void raster_wave(const ViewParams& V, uint64_t* tile,
         if (bw <= kTilePixels && bh <= (kTilePixels >> lg)) {
             const uint32_t lane = threadIdx.x & (kWave - 1);
             const uint32_t count = bh << lg;
-            for (uint32_t k = lane; k < count; k += kWave) tile[k] = ~0ull;
-            wave_sync();
             if (has)
                 raster_rows(r, fast, id, slot, step, ((uint32_t)(r.y - y0) << lg) + (uint32_t)(r.x - x0), 1u << lg,
                             [&](uint32_t at, uint64_t packed) {
                                 atomicMin((unsigned long long*)(tile + at), (unsigned long long)packed);
                             });
             wave_sync();
-            const uint32_t origin = (uint32_t)x0 + (uint32_t)V.W * (uint32_t)y0;
+            const uint32_t W = (uint32_t)V.W, mask = (1u << lg) - 1u;
+            uint32_t at = (uint32_t)x0 + W * (uint32_t)y0 + (lane & mask) + W * (lane >> lg);
             for (uint32_t k = lane; k < count; k += kWave) {
                 const uint64_t v = tile[k];
-                if (v != ~0ull)
-                    atomic_min_fb(V.fb, origin + (k & ((1u << lg) - 1u)) + (uint32_t)V.W * (k >> lg), v);
+                tile[k] = ~0ull;
+                if (v != ~0ull) atomic_min_fb(V.fb, at, v);
+                // 64 samples on: whole rows, or part of a wider one
+                if (lg <= 6u) at += W << (6u - lg);
+                else at += ((k + kWave) & mask) >= kWave ? kWave : W + kWave - (mask + 1u);
             }
             wave_sync();
             return;
@@ -1517,6 +1524,7 @@ __global__ __launch_bounds__(256) void k_stage1_coarse(RasterParams P) {
     __shared__ uint64_t tiles[256 / kWave][kTilePixels];
     __shared__ uint32_t queued[256 / kWave], queueBase;
     uint64_t* tile = tiles[threadIdx.x / kWave];
+    tile_clear(tile);
     const ViewParams V0 = kconst(P.views)[0];
     const auto transforms = kconst(V0.transforms);
     const uint32_t shift = P.splitShift;
@@ -1611,6 +1619,8 @@ struct RunLayout {
 struct RunBatch {
     uint32_t unit, strip, row, col, rowEnd;
     uint32_t inside;    // the unit lies inside the view (kUnitInside or 0)
+    uint32_t view;      // listed: the view to draw it into
+    uint32_t row0;      // squares: the unit's first row (`row` then counts its squares)
 };
 
 // Top bit of a listed unit (k_cull_units): all of it lies inside the view.
@@ -1630,6 +1640,41 @@ __device__ __forceinline__ void run_bounds(const S1Item& it, const RunLayout& L,
     end = uni((uint32_t)min(start + w, (uint64_t)it.numTriangles));
 }
 
+// Squares (k_stage1_pairs of several views): the wave's 128 triangles are 8
+// rows of 8 pairs, so that what it draws lies close together on the screen.
+// `base` is the square's first triangle, `end` its rows << 8 | its triangles
+// per row.
+constexpr uint32_t kSquareCols = 16;     // triangles
+static_assert(2u * kWave / kSquareCols == kUnitRows, "a unit holds as many squares as rows");
+
+__device__ __forceinline__ void square_bounds(const S1Item& it, const RunLayout& L, const RunBatch& b, uint32_t& base,
+                                              uint32_t& end) {
+    const uint64_t x = (uint64_t)b.strip * (2u * kWave) + (uint64_t)b.row * kSquareCols;
+    const uint64_t start = (uint64_t)b.row0 * L.rowTris + x;
+    const uint32_t rows = b.row0 < L.rows ? min(kUnitRows, L.rows - b.row0) : 0u;
+    const uint32_t cols = x < L.rowTris ? (uint32_t)min((uint64_t)kSquareCols, (uint64_t)L.rowTris - x) : 0u;
+    base = uni((uint32_t)min(start, (uint64_t)it.numTriangles));
+    end = uni(rows << 8 | cols);
+}
+
+// The lane's first triangle of a batch and how many of its two there are.
+template <bool SQUARE>
+__device__ __forceinline__ uint32_t lane_tris(const S1Item& it, uint32_t rowTris, uint32_t base, uint32_t end,
+                                              uint32_t lane, uint32_t& count) {
+    if constexpr (!SQUARE) {
+        const uint32_t t = base + 2u * lane;
+        count = t < end ? min(end - t, 2u) : 0u;
+        return t;
+    } else {
+        const uint32_t row = lane / (kSquareCols / 2u), col = 2u * (lane % (kSquareCols / 2u));
+        const uint64_t t = base + (uint64_t)row * rowTris + col;
+        const uint32_t cols = end & 0xFFu;
+        count = row < (end >> 8) && col < cols && t < it.numTriangles
+                    ? min(min(cols - col, it.numTriangles - (uint32_t)t), 2u) : 0u;
+        return (uint32_t)min(t, (uint64_t)it.numTriangles);
+    }
+}
+
 // First batch of unit u.
 __device__ __forceinline__ RunBatch run_first(const RunLayout& L, uint32_t u) {
     const uint32_t rel = u - L.firstUnit;
@@ -1637,6 +1682,8 @@ __device__ __forceinline__ RunBatch run_first(const RunLayout& L, uint32_t u) {
     const uint32_t g = rel - s * L.unitSegs;
     RunBatch b;
     b.inside = 0u;
+    b.view = 0u;
+    b.row0 = 0u;
     b.unit = uni(u);
     b.strip = s;
     b.col = 0u;
@@ -1672,7 +1719,7 @@ constexpr uint32_t kStaticPartShift = 2;
 
 struct UnitSource {
     uint32_t* claims;
-    const uint32_t* list;
+    const uint64_t* list;  // view << 32 | kUnitInside or 0 | unit
     uint32_t total;        // parts
     uint32_t partShift;
     uint32_t waves;        // of the grid
@@ -1683,7 +1730,7 @@ struct UnitSource {
     __device__ __forceinline__ uint64_t part_of(uint32_t k) const {
         if (k >= total) return ~0ull;
         if (!LISTED) return k;
-        return ((uint64_t)kconst(list)[k >> partShift] << 8) | (k & ((1u << partShift) - 1u));
+        return (kconst(list)[k >> partShift] << 8) | (k & ((1u << partShift) - 1u));
     }
     template <bool LISTED>
     static __device__ __forceinline__ uint32_t unit_of(uint64_t part) {
@@ -1706,10 +1753,18 @@ struct UnitSource {
 };
 
 // First batch of a part.
-template <bool LISTED>
+template <bool LISTED, bool SQUARE>
 __device__ __forceinline__ RunBatch part_first(const RunLayout& L, uint64_t part, uint32_t partShift) {
     RunBatch b = run_first(L, UnitSource::unit_of<LISTED>(part));
     b.inside = LISTED ? uni((uint32_t)(part >> 8) & kUnitInside) : 0u;
+    b.view = LISTED ? uni((uint32_t)(part >> 40)) : 0u;
+    if constexpr (SQUARE) {
+        const uint32_t n = kUnitRows >> partShift;      // squares of the part
+        b.row0 = b.row;
+        b.row = uni(((uint32_t)part & 0xFFu) * n);
+        b.rowEnd = uni(b.row + n);
+        return b;
+    }
     if (LISTED && partShift > 0u) {
         const uint32_t rows = kUnitRows >> partShift;
         b.row = uni(b.row + ((uint32_t)part & 0xFFu) * rows);
@@ -1725,7 +1780,7 @@ __device__ __forceinline__ RunBatch part_first(const RunLayout& L, uint64_t part
 // the first row of a newly claimed part of the same item; more = 0 when the
 // claimed part lies past the item (left in `pending` for the next pass; the
 // batch returned is then `a` again, a valid address to reload).
-template <bool LISTED>
+template <bool LISTED, bool SQUARE>
 __device__ __forceinline__ RunBatch run_next(const RunLayout& L, UnitSource& U, uint32_t iend, const RunBatch& a,
                                              uint32_t& more, uint64_t& pending) {
     more = 1u;
@@ -1742,7 +1797,7 @@ __device__ __forceinline__ RunBatch run_next(const RunLayout& L, UnitSource& U, 
     }
     const uint64_t part = U.next<LISTED>();
     const uint32_t u = UnitSource::unit_of<LISTED>(part);
-    if (part != ~0ull && u >= L.firstUnit && u < iend) return part_first<LISTED>(L, part, U.partShift);
+    if (part != ~0ull && u >= L.firstUnit && u < iend) return part_first<LISTED, SQUARE>(L, part, U.partShift);
     pending = part;
     more = 0u;
     return a;
@@ -1768,9 +1823,9 @@ __device__ __forceinline__ void pair_pu16_range(const S1Item& it, uint32_t base,
     avail = (uint32_t)min(need, numWords - firstWord);
 }
 
-template <bool PU16>
-__device__ __forceinline__ void pair_indices(const S1Item& it, uint32_t base, uint32_t end, uint32_t lane,
-                                             uint32_t (&I)[6]) {
+template <bool PU16, bool SQUARE>
+__device__ __forceinline__ void pair_indices(const S1Item& it, uint32_t rowTris, uint32_t base, uint32_t end,
+                                             uint32_t lane, uint32_t (&I)[6]) {
 #if defined(__HIP_DEVICE_COMPILE__)
     __amdgpu_buffer_rsrc_t rs;
     if constexpr (PU16) {
@@ -1780,18 +1835,23 @@ __device__ __forceinline__ void pair_indices(const S1Item& it, uint32_t base, ui
         if (it.bits == 0u || it.bits > 32u) avail = 0u;     // BitEdit::readU32 reads nothing
         rs = buffer_rsrc(it.indices + firstWord, 4u * avail);
     } else {
-        rs = buffer_rsrc(it.indices + 3ull * base, 12u * (end - base));
+        // squares: up to the item's end (words past it read as zero)
+        const uint64_t tris = SQUARE ? (uint64_t)it.numTriangles - base : (uint64_t)(end - base);
+        rs = buffer_rsrc(it.indices + 3ull * base, (uint32_t)min(12ull * tris, 0xFFFFFFFCull));
     }
-    const uint4 v = buffer_load_u4(rs, 24u * lane);
-    const uint2 w = buffer_load_u2(rs, 24u * lane + 16u);
+    uint32_t count;
+    const uint32_t first = SQUARE ? lane_tris<SQUARE>(it, rowTris, base, end, lane, count) : base + 2u * lane;
+    const uint32_t at = SQUARE ? 12u * (first - base) : 24u * lane;   // (squares: below 2^32, see plan_draw)
+    const uint4 v = buffer_load_u4(rs, at);
+    const uint2 w = buffer_load_u2(rs, at + 16u);
     I[0] = v.x; I[1] = v.y; I[2] = v.z; I[3] = v.w; I[4] = w.x; I[5] = w.y;
     if (!PU16 && it.indexMask == 0u) {          // wave-uniform; no loads in this branch
-        const uint32_t t = min(base + 2u * lane, it.numTriangles - 1u), t1 = min(t + 1u, it.numTriangles - 1u);
+        const uint32_t t = min(first, it.numTriangles - 1u), t1 = min(t + 1u, it.numTriangles - 1u);
         I[0] = 3u * t; I[1] = 3u * t + 1u; I[2] = 3u * t + 2u;
         I[3] = 3u * t1; I[4] = 3u * t1 + 1u; I[5] = 3u * t1 + 2u;
     }
 #else
-    (void)it; (void)base; (void)end; (void)lane;
+    (void)it; (void)rowTris; (void)base; (void)end; (void)lane;
     for (int j = 0; j < 6; j++) I[j] = 0u;
 #endif
 }
@@ -1845,13 +1905,12 @@ __device__ __forceinline__ void pair_pu16_decode(const S1Item& it, uint32_t base
 // pu16_vertex_decode.
 template <bool PU16>
 __device__ __forceinline__ uint32_t pair_vertices(const S1Item& it, uint32_t base, uint32_t end, uint32_t lane,
-                                                  uint32_t* words, uint32_t (&I)[6], f3 (&S)[6]) {
+                                                  uint32_t count, uint32_t* words, uint32_t (&I)[6], f3 (&S)[6]) {
     if constexpr (PU16) pair_pu16_decode(it, base, end, lane, words, I);
-    const uint32_t rel = 2u * lane;
-    if (base + rel >= end) {
+    if (count == 0u) {
         I[1] = I[2] = I[0];
     }
-    if (base + rel + 1u >= end) {
+    if (count < 2u) {
         I[3] = I[0];
         I[4] = I[2];
         I[5] = I[1];
@@ -1886,9 +1945,10 @@ __device__ __forceinline__ uint32_t pair_vertices(const S1Item& it, uint32_t bas
 // s1_sweep: while batch i is drawn, the gathers of batch i+1 and the index
 // loads of batch i+2 are in flight.  Units (strip, group of rows) are dealt
 // to the workgroups by P.order as s1_range deals batches; a workgroup walks
-// its unit's rows in turn.  body(it, base, end, S, pattern, inside, last)
-// draws one batch; `last` marks the last one of a pass over an item.
-template <bool PU16, bool LISTED, typename Body>
+// its unit's rows in turn.  body(it, t, count, S, pattern, inside,
+// view, last) draws one batch, lane by lane `count` triangles from t; `last` marks the last one of a pass over an item, or
+// before another view's.
+template <bool PU16, bool LISTED, bool SQUARE, typename Body>
 __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* words, Body&& body) {
     const uint32_t numUnits = P.batchCount ? *kconst(P.batchCount) : P.numBatches;
     const uint32_t lane = threadIdx.x & (kWave - 1);
@@ -1920,25 +1980,32 @@ __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* 
         L.firstUnit = it.firstBatch;
         const uint32_t iend = it.endBatch;
         uint64_t pending = ~0ull;
+        const auto bounds = [&](const RunBatch& b, uint32_t& base, uint32_t& end) __attribute__((always_inline)) {
+            if constexpr (SQUARE) square_bounds(it, L, b, base, end);
+            else run_bounds(it, L, b, base, end);
+        };
+        uint32_t n0, n1;
         uint32_t base0, end0, base1, end1, base2, end2;
-        const RunBatch b0 = part_first<LISTED>(L, part, U.partShift);
-        run_bounds(it, L, b0, base0, end0);
+        const RunBatch b0 = part_first<LISTED, SQUARE>(L, part, U.partShift);
+        bounds( b0, base0, end0);
         uint32_t I[6], J[6];
-        pair_indices<PU16>(it, base0, end0, lane, I);
+        pair_indices<PU16, SQUARE>(it, L.rowTris, base0, end0, lane, I);
         uint32_t more1;
-        RunBatch b1 = run_next<LISTED>(L, U, iend, b0, more1, pending);
-        run_bounds(it, L, b1, base1, end1);
-        pair_indices<PU16>(it, base1, end1, lane, J);
+        RunBatch b1 = run_next<LISTED, SQUARE>(L, U, iend, b0, more1, pending);
+        bounds( b1, base1, end1);
+        pair_indices<PU16, SQUARE>(it, L.rowTris, base1, end1, lane, J);
         f3 S[6];
-        uint32_t pat = pair_vertices<PU16>(it, base0, end0, lane, words, I, S);
-        uint32_t inside = b0.inside;
+        (void)lane_tris<SQUARE>(it, L.rowTris, base0, end0, lane, n0);
+        uint32_t pat = pair_vertices<PU16>(it, base0, end0, lane, n0, words, I, S);
+        uint32_t inside = b0.inside, view = b0.view;
         for (;;) {
             f3 Sn[6];
-            const uint32_t patN = pair_vertices<PU16>(it, base1, end1, lane, words, J, Sn);
+            (void)lane_tris<SQUARE>(it, L.rowTris, base1, end1, lane, n1);
+            const uint32_t patN = pair_vertices<PU16>(it, base1, end1, lane, n1, words, J, Sn);
             uint32_t more2 = 0u;
-            const RunBatch b2 = more1 ? run_next<LISTED>(L, U, iend, b1, more2, pending) : b1;
-            run_bounds(it, L, b2, base2, end2);
-            pair_indices<PU16>(it, base2, end2, lane, J);
+            const RunBatch b2 = more1 ? run_next<LISTED, SQUARE>(L, U, iend, b1, more2, pending) : b1;
+            bounds( b2, base2, end2);
+            pair_indices<PU16, SQUARE>(it, L.rowTris, base2, end2, lane, J);
             if constexpr (PU16) {
                 #pragma unroll
                 for (int j = 0; j < 4; j++) S[j] = pu16_vertex_decode(it, S[j]);
@@ -1947,9 +2014,11 @@ __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* 
                     S[5] = pu16_vertex_decode(it, S[5]);
                 }
             }
-            body(it, base0, end0, S, pat, inside != 0u, !more1);
+            const uint32_t t0 = lane_tris<SQUARE>(it, L.rowTris, base0, end0, lane, n0);
+            body(it, t0, n0, S, pat, inside != 0u, view, !more1 || (LISTED && b1.view != view));
             if (!more1) break;
             inside = b1.inside;
+            view = b1.view;
             base0 = base1;
             end0 = end1;
             b1 = b2;
@@ -2023,10 +2092,11 @@ __device__ __forceinline__ uint32_t mask_rank(uint64_t mask) {
 }
 
 // The triangles that the filter left, per wave: fewer than 64 from earlier
-// batches and up to 128 of this one.
+// batches and up to 128 (of half a batch, 64) more.
+template <uint32_t CAP>
 struct LeftTris {
-    float p[9][3 * kWave];
-    uint32_t tri[3 * kWave];
+    float p[9][CAP];
+    uint32_t tri[CAP];
 
     __device__ __forceinline__ void put(uint32_t at, uint32_t t, const f3& a, const f3& b, const f3& c) {
         p[0][at] = a.x; p[1][at] = a.y; p[2][at] = a.z;
@@ -2044,8 +2114,9 @@ struct LeftTris {
 
 }  // namespace
 
-// Stage 1 over pairs of consecutive triangles for draws of one view whose
-// items are drawn over few instances (the others take k_stage1).
+// Stage 1 over pairs of consecutive triangles for draws whose items are drawn
+// over few instances (the others take k_stage1 and k_stage1_views): of one
+// view, or (VIEWS, listed) of the views that k_cull_units lists each unit for.
 //
 // Bound by VALU issue before it is by memory: the exact code takes about 280
 // instructions per 64 triangles, and most of a large mesh's triangles hold no
@@ -2058,33 +2129,52 @@ struct LeftTris {
 // MB in place of 520 and wait (143 us against 134).
 // Stage 1 of that terrain 195 -> 130 us (VALU instructions 112 M -> 50 M, 4.0
 // TB/s fetched), of the 400 M-triangle one's 1.5% in view 79 -> 62.
-template <int BLOCK, bool PU16, bool LISTED>
-__global__ __launch_bounds__(BLOCK) void k_stage1_pairs(RasterParams P) {
-    const ViewParams V0 = kconst(P.views)[0];
-    const auto transforms = kconst(V0.transforms);
+//
+// Several views: a unit is drawn once for every view that may see it, where
+// k_stage1_views tests every 64 triangles against every view.  Their triangles
+// are larger too, so that the 64-bit atomics to memory weigh in (in rows of 64
+// pairs, lane by lane, 71 M requests and 3.6 ms for 64 views, of which 2.3
+// remain when no sample is sent).  So a batch is a square of 8 rows of 8 pairs,
+// which fits the LDS tile of raster_wave: 43 M requests, 3.4 ms, against 4.3
+// of k_stage1_views (VALU instructions 2394 M -> 1914 M).  IX_PU16 streams are
+// cut per row, so they keep the rows and the lane's own atomics.
+template <int BLOCK, bool PU16, bool LISTED, bool VIEWS>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(PU16 || VIEWS ? 1 : 5))) void k_stage1_pairs(RasterParams P) {
     uint32_t* words = nullptr;
     if constexpr (PU16) {
         __shared__ __align__(16) uint32_t pairWords[BLOCK / kWave][kPairPu16Words];
         words = pairWords[threadIdx.x / kWave];
     }
-    __shared__ LeftTris leftTris[BLOCK / kWave];
-    LeftTris& left = leftTris[threadIdx.x / kWave];
-    const FilterView F = filter_view(V0);
+    // of several views, in squares: the wave's minima go through an LDS tile
+    constexpr bool SQUARE = VIEWS && !PU16;
+    constexpr uint32_t CAP = SQUARE ? 2u * kWave : 3u * kWave;
+    __shared__ LeftTris<CAP> leftTris[BLOCK / kWave];
+    auto& left = leftTris[threadIdx.x / kWave];
+    uint64_t* tile = nullptr;
+    if constexpr (SQUARE) {
+        __shared__ uint64_t tiles[BLOCK / kWave][kTilePixels];
+        tile = tiles[threadIdx.x / kWave];
+        tile_clear(tile);
+    }
+    const ViewParams V0 = kconst(P.views)[0];
     uint32_t queued = 0;
-    s1_pairs_sweep<PU16, LISTED>(P, words, [&](const S1Item& it, uint32_t base, uint32_t end, const f3 (&S)[6],
-                                               uint32_t pat, bool inside, bool last) __attribute__((always_inline)) {
+    s1_pairs_sweep<PU16, LISTED, SQUARE>(P, words, [&](const S1Item& it, uint32_t ta, uint32_t count, const f3 (&S)[6],
+                                                       uint32_t pat, bool inside, uint32_t view, bool last)
+                                                       __attribute__((always_inline)) {
+        const ViewParams V = VIEWS ? kconst(P.views)[view] : V0;
+        const FilterView F = filter_view(V);
         const uint32_t lane = threadIdx.x & (kWave - 1);
-        const uint32_t ta = base + 2u * lane, tb = ta + 1u;
         for (uint32_t j = 0; j < it.instCount; j++) {
             const uint32_t inst = it.instOffset + j;
-            const auto T = transforms + inst;
+            const auto T = kconst(V.transforms) + inst;
             float m[16];
             #pragma unroll
             for (int e = 0; e < 16; e++) m[e] = T->m[e];
             const bool flip = T->flip != 0u;
+            const bool skip = VIEWS && T->skip != 0u;   // dropped from this view
             const FV v0 = filter_vertex(F, m, S[0]), v1 = filter_vertex(F, m, S[1]), v2 = filter_vertex(F, m, S[2]),
                      v3 = filter_vertex(F, m, S[3]);
-            const bool keepA = ta < end && !filter_culls(F, LISTED && inside, v0, v1, v2);
+            const bool keepA = count > 0u && !skip && !filter_culls(F, LISTED && inside, v0, v1, v2);
             FV b0 = v0, b1 = v3, b2 = v1;                     // kPairFan: (A.a, n, A.b)
             if (pat == kPairGrid) {                           // (A.a, A.c, n)
                 b1 = v2;
@@ -2094,30 +2184,50 @@ __global__ __launch_bounds__(BLOCK) void k_stage1_pairs(RasterParams P) {
                 b1 = filter_vertex(F, m, S[4]);
                 b2 = filter_vertex(F, m, S[5]);
             }
-            const bool keepB = tb < end && !filter_culls(F, LISTED && inside, b0, b1, b2);
+            const bool keepB = count > 1u && !skip && !filter_culls(F, LISTED && inside, b0, b1, b2);
+            // (in squares a pair's two triangles lie side by side, and half the
+            // wave goes at a time where the batch may overflow the queue)
             const uint64_t ma = __ballot(keepA), mb = __ballot(keepB);
-            if (keepA) left.put(queued + mask_rank(ma), ta, S[0], S[1], S[2]);
-            queued += (uint32_t)__popcll(ma);
-            if (keepB) {
-                const uint32_t at = queued + mask_rank(mb);
-                if (pat == kPairGrid) left.put(at, tb, S[0], S[2], S[3]);
-                else if (pat == kPairFan) left.put(at, tb, S[0], S[3], S[1]);
-                else left.put(at, tb, S[3], S[4], S[5]);
-            }
-            queued += (uint32_t)__popcll(mb);
-            // what is left of an instance, or of the pass over an item, is drawn at its end
-            const bool all = last || it.instCount > 1u;
-            while (queued >= kWave || (all && queued > 0u)) {
-                const uint32_t n = min(queued, (uint32_t)kWave);
-                queued -= n;
-                wave_sync();
-                f3 A, B, C;
-                const uint32_t t = left.get(queued + min(lane, n - 1u), A, B, C);
-                wave_sync();
-                const uint64_t id = it.cumm + (uint64_t)t + (uint64_t)(j * it.numTriangles);
-                if (lane < n)
-                    stage1_triangle(P, V0, m, flip, A, B, C, id, ((uint64_t)inst << 32) | t,
-                                    item_cull_order(P, it.instCount));
+            const bool halves = CAP < 3u * kWave && queued + (uint32_t)(__popcll(ma) + __popcll(mb)) > CAP;
+            #pragma nounroll
+            for (uint32_t part = halves ? 0u : 1u; part < 2u; part++) {
+                const uint64_t sel = !halves ? ~0ull : part ? 0xFFFFFFFF00000000ull : 0xFFFFFFFFull;
+                const bool mine = !halves || lane / (kWave / 2u) == part;
+                const uint32_t at = queued + mask_rank(ma & sel) + (SQUARE ? mask_rank(mb & sel) : 0u);
+                if (keepA && mine) left.put(at, ta, S[0], S[1], S[2]);
+                if (keepB && mine) {
+                    const uint32_t atB = SQUARE ? at + (keepA ? 1u : 0u)
+                                                : queued + (uint32_t)__popcll(ma) + mask_rank(mb);
+                    if (pat == kPairGrid) left.put(atB, ta + 1u, S[0], S[2], S[3]);
+                    else if (pat == kPairFan) left.put(atB, ta + 1u, S[0], S[3], S[1]);
+                    else left.put(atB, ta + 1u, S[3], S[4], S[5]);
+                }
+                queued += (uint32_t)(__popcll(ma & sel) + __popcll(mb & sel));
+                // what is left of an instance, a pass or a view is drawn at its end
+                const bool all = (last || it.instCount > 1u) && part == 1u;
+                while (queued >= kWave || (all && queued > 0u)) {
+                    const uint32_t n = min(queued, (uint32_t)kWave);
+                    queued -= n;
+                    wave_sync();
+                    f3 A, B, C;
+                    const uint32_t t = left.get(queued + min(lane, n - 1u), A, B, C);
+                    wave_sync();
+                    const uint64_t id = it.cumm + (uint64_t)t + (uint64_t)(j * it.numTriangles);
+                    const uint64_t entry = ((uint64_t)((view << kViewShift) | inst) << 32) | t;
+                    const uint32_t cullOrder = item_cull_order(P, it.instCount);
+                    if constexpr (SQUARE) {
+                        RasterTri rt;
+                        S1Result todo = S1_NONE;
+                        if (lane < n) todo = stage1_core<true>(P, V, m, flip, A, B, C, id, entry, cullOrder, &rt);
+                        if (todo == S1_QUEUE) {
+                            const uint32_t slot = atomicAdd(P.ctrNontrivial, 1u);
+                            if (slot < P.ntCap) P.nontrivial[slot] = entry;
+                        }
+                        raster_wave(V, tile, rt, todo == S1_RASTER, id, 0u, 1u);
+                    } else {
+                        if (lane < n) stage1_triangle(P, V, m, flip, A, B, C, id, entry, cullOrder);
+                    }
+                }
             }
         }
     });
@@ -2193,7 +2303,9 @@ __global__ __launch_bounds__(256) void k_unit_bounds(DrawItem it, uint32_t numUn
 
 constexpr uint32_t kCullChunk = 1024;    // units per workgroup, one per lane
 
-// Lists the units of a single-view draw that the view may see (view_may_see:
+// Lists the units of a draw that a view may see (workgroup c * views + v:
+// view v, chunk c; the views of a chunk follow each other, so that those that draw a
+// unit find it in the caches; view_may_see:
 // a unit is dropped only when every triangle in it is culled by its own exact
 // tests), and marks those wholly inside it (kUnitInside; every instance's,
 // where the item has several).  One append per workgroup of 1024 units: the
@@ -2206,10 +2318,11 @@ __global__ __launch_bounds__(1024) void k_cull_units(RasterParams P) {
     __shared__ uint32_t listBase;
     const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const uint32_t numUnits = P.numBatches;
-    const uint32_t u = blockIdx.x * kCullChunk + threadIdx.x;
+    const uint32_t chunk = blockIdx.x / P.numViews, view = blockIdx.x - chunk * P.numViews;
+    const uint32_t u = chunk * kCullChunk + threadIdx.x;
     // the chunk's first and last item: usually the same one
-    const uint32_t first = find_item(P, blockIdx.x * kCullChunk);
-    uint32_t lo = first, hi = find_item(P, min(numUnits, (blockIdx.x + 1u) * kCullChunk) - 1u);
+    const uint32_t first = find_item(P, chunk * kCullChunk);
+    uint32_t lo = first, hi = find_item(P, min(numUnits, (chunk + 1u) * kCullChunk) - 1u);
     bool keep = false, inside = false;
     if (u < numUnits) {
         while (lo < hi) {
@@ -2231,8 +2344,8 @@ __global__ __launch_bounds__(1024) void k_cull_units(RasterParams P) {
                 keep = false;
                 inside = true;
                 for (uint32_t j = 0; j < it.instCount; j++) {
-                    const ViewCull c = lane_view_cull(P, 0u, it.instOffset + j);
-                    keep = keep || view_may_see(c, box);
+                    const ViewCull c = lane_view_cull(P, view, it.instOffset + j);
+                    keep = keep || (!c.skip && view_may_see(c, box));
                     inside = inside && view_inside(c, box);
                 }
             }
@@ -2257,7 +2370,7 @@ __global__ __launch_bounds__(1024) void k_cull_units(RasterParams P) {
     if (keep) {
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(kept >> 32),
                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0u));
-        P.units[listBase + counts[wave] + rank] = u | (inside ? kUnitInside : 0u);
+        P.units[listBase + counts[wave] + rank] = ((uint64_t)view << 32) | u | (inside ? kUnitInside : 0u);
     }
 }
 
@@ -3479,19 +3592,29 @@ hipError_t launch_stage1_coarse(const RasterParams& P, uint32_t grid, bool pu16,
     return hipGetLastError();
 }
 
+namespace {
+
+template <bool PU16>
+void launch_pairs(const RasterParams& P, uint32_t grid, bool listed, hipStream_t stream) {
+    if (listed && P.numViews > 1u)
+        hipLaunchKernelGGL((k_stage1_pairs<256, PU16, true, true>), dim3(grid), dim3(256), 0, stream, P);
+    else if (listed) hipLaunchKernelGGL((k_stage1_pairs<256, PU16, true, false>), dim3(grid), dim3(256), 0, stream, P);
+    else hipLaunchKernelGGL((k_stage1_pairs<256, PU16, false, false>), dim3(grid), dim3(256), 0, stream, P);
+}
+
+}  // namespace
+
 hipError_t launch_stage1_pairs(const RasterParams& P, uint32_t block, uint32_t grid, bool pu16, bool listed,
                                hipStream_t stream) {
-    if (block != 256) return hipErrorInvalidValue;
-    if (pu16 && listed) hipLaunchKernelGGL((k_stage1_pairs<256, true, true>), dim3(grid), dim3(256), 0, stream, P);
-    else if (pu16) hipLaunchKernelGGL((k_stage1_pairs<256, true, false>), dim3(grid), dim3(256), 0, stream, P);
-    else if (listed) hipLaunchKernelGGL((k_stage1_pairs<256, false, true>), dim3(grid), dim3(256), 0, stream, P);
-    else hipLaunchKernelGGL((k_stage1_pairs<256, false, false>), dim3(grid), dim3(256), 0, stream, P);
+    if (block != 256 || (P.numViews > 1u && !listed)) return hipErrorInvalidValue;
+    if (pu16) launch_pairs<true>(P, grid, listed, stream);
+    else launch_pairs<false>(P, grid, listed, stream);
     return hipGetLastError();
 }
 
 hipError_t launch_cull_units(const RasterParams& P, hipStream_t stream) {
-    const uint32_t blocks = (P.numBatches + kCullChunk - 1u) / kCullChunk;
-    hipLaunchKernelGGL(k_cull_units, dim3(blocks), dim3(1024), 0, stream, P);
+    const uint32_t chunks = (P.numBatches + kCullChunk - 1u) / kCullChunk;
+    hipLaunchKernelGGL(k_cull_units, dim3(chunks * P.numViews), dim3(1024), 0, stream, P);
     return hipGetLastError();
 }
 

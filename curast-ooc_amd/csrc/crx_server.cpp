@@ -52,6 +52,7 @@
 
 #include "crx_device.h"
 #include "crx_host.h"
+#include "crx_internal.h"
 
 using namespace crx;
 
@@ -67,6 +68,7 @@ struct Node {
     crx_mat4 world{};
     uint64_t cumm = 0;
     bool wantResident = false;
+    uint32_t rowTris = 0;         // row length of the index order (0: none found)
     // cache state (guarded by the cache mutex)
     int slot = -1;
     uint32_t pins = 0;
@@ -139,6 +141,10 @@ struct crx_server {
     char* cache = nullptr;
     size_t slotBytes = 0;
     uint32_t numSlots = 0;
+    // boxes of the stage-1 units of each slot's node (slotUnits per slot),
+    // computed after the node's upload; null when they could not be allocated
+    UnitBox* boxes = nullptr;
+    uint64_t slotUnits = 0;
     std::vector<int> slotNode;      // node in each slot, -1 = free
     std::vector<uint32_t> slotReaders;   // lanes (bit mask) whose reads of the slot's node may be in flight
     hipStream_t upload = nullptr;
@@ -190,6 +196,9 @@ struct crx_server {
 
 namespace {
 
+// Triangles of a node whose index order is searched for its row length.
+constexpr uint64_t kRowWindow = 1u << 13;
+
 size_t node_bytes(const Node& n) {
     return align_up(12ull * n.numVertices, kAlign) + align_up(12ull * n.numTriangles, kAlign) +
            align_up(4ull * n.numVertices, kAlign);
@@ -202,6 +211,12 @@ void slot_pointers(crx_server* s, const Node& n, float** pos, uint32_t** idx, ui
     *idx = reinterpret_cast<uint32_t*>(base + align_up(12ull * n.numVertices, kAlign));
     *col = reinterpret_cast<uint32_t*>(base + align_up(12ull * n.numVertices, kAlign) +
                                        align_up(12ull * n.numTriangles, kAlign));
+}
+
+// Stage-1 item of a node's geometry in the default walk, and its number of units.
+uint64_t node_units(const Node& n, DrawItem* it) {
+    it->numTriangles = n.numTriangles;
+    return pair_layout(*it, n.rowTris, kUnitRows, 1u);
 }
 
 // Copies node `id` into `slot` on `stream` (the upload stream by default)
@@ -224,6 +239,15 @@ crx_status upload_node(crx_server* s, uint32_t id, int slot, hipStream_t stream 
         CRX_HIP(hipMemcpyAsync(idx, n.hidx, 12ull * n.numTriangles, hipMemcpyHostToDevice, stream));
     if (n.hcol && n.numVertices)
         CRX_HIP(hipMemcpyAsync(col, n.hcol, 4ull * n.numVertices, hipMemcpyHostToDevice, stream));
+    if (s->boxes && n.numTriangles) {
+        DrawItem it{};
+        const uint64_t units = node_units(n, &it);
+        it.indices = n.hidx ? idx : reinterpret_cast<const uint32_t*>(pos);
+        it.indexMask = n.hidx ? 0xFFFFFFFFu : 0u;
+        it.positions = pos;
+        it.numVertices = n.numVertices;
+        CRX_HIP(launch_unit_bounds(it, false, (uint32_t)units, s->boxes + (size_t)slot * s->slotUnits, stream));
+    }
     if (!n.ready) CRX_HIP(hipEventCreateWithFlags(&n.ready, hipEventDisableTiming));
     CRX_HIP(hipEventRecord(n.ready, stream));
     s->statUploads++;
@@ -424,14 +448,30 @@ crx_cmesh node_cmesh(crx_server* s, uint32_t id, uint32_t k) {
     return m;
 }
 
-// CMesh records of the pinned nodes `ids`, and `stream` ordered after their uploads.
+// Unit boxes and row lengths of the nodes of a draw.
+struct NodeBounds {
+    std::vector<const UnitBox*> boxes;
+    std::vector<uint32_t> rows;
+    DrawBounds bounds() const {
+        DrawBounds b;
+        b.boxes = boxes.data();
+        b.rows = rows.data();
+        return b;
+    }
+};
+
+// CMesh records (and unit boxes) of the pinned nodes `ids`, and `stream` ordered after their uploads.
 crx_status pinned_cmeshes(crx_server* s, const std::vector<uint32_t>& ids, hipStream_t stream,
-                          std::vector<crx_cmesh>* inst) {
+                          std::vector<crx_cmesh>* inst, NodeBounds* nb) {
     std::lock_guard<std::mutex> lk(s->cacheMu);   // slot pointers are stable while pinned
     inst->resize(ids.size());
+    nb->boxes.resize(ids.size());
+    nb->rows.resize(ids.size());
     for (uint32_t k = 0; k < ids.size(); k++) {
         const Node& n = s->nodes[ids[k]];
         (*inst)[k] = node_cmesh(s, ids[k], k);
+        nb->boxes[k] = s->boxes ? s->boxes + (size_t)n.slot * s->slotUnits : nullptr;
+        nb->rows[k] = n.rowTris;
         if (n.ready) CRX_HIP(hipStreamWaitEvent(stream, n.ready, 0));
     }
     return CRX_OK;
@@ -508,6 +548,7 @@ crx_status draw_group(crx_server* s, crx_server::Lane& lane, const std::vector<R
         return anySkip && V > 1;
     };
     std::vector<crx_cmesh> inst;
+    NodeBounds nb;
 
     if (need.size() <= s->numSlots) {
         uint32_t up = 0;
@@ -515,7 +556,7 @@ crx_status draw_group(crx_server* s, crx_server::Lane& lane, const std::vector<R
         *uploads += up;
         crx_status st = CRX_OK;
         do {
-            st = pinned_cmeshes(s, need, lane.stream, &inst);
+            st = pinned_cmeshes(s, need, lane.stream, &inst, &nb);
             if (st != CRX_OK) break;
             const uint32_t U = (uint32_t)need.size();
             const bool useSkip = lists(need);
@@ -536,6 +577,7 @@ crx_status draw_group(crx_server* s, crx_server::Lane& lane, const std::vector<R
             ex.afterStages = s->cfg.resolve ? &resolve : nullptr;
             ex.prefix = s->cfg.resolve != 0;
             ex.earlyReturn = true;   // lane_finish waits for the resolve
+            ex.bounds = nb.bounds();
             st = draw_views(lane.ctx, inst.data(), U, inst.data(), U, xf.data(), targets.data(), V, 0, lane.stream, &ds,
                             ex);
         } while (false);
@@ -562,7 +604,7 @@ crx_status draw_group(crx_server* s, crx_server::Lane& lane, const std::vector<R
         uint32_t up = 0;
         CRX_TRY(acquire_nodes(s, ids, &up));
         *uploads += up;
-        crx_status st = pinned_cmeshes(s, ids, lane.stream, &inst);
+        crx_status st = pinned_cmeshes(s, ids, lane.stream, &inst, &nb);
         if (st == CRX_OK) {
             const uint32_t U = (uint32_t)ids.size();
             if (!resolvePass) {
@@ -570,6 +612,7 @@ crx_status draw_group(crx_server* s, crx_server::Lane& lane, const std::vector<R
                 DrawExtras ex;
                 ex.skip = useSkip ? skip.data() : nullptr;
                 ex.earlyReturn = true;
+                ex.bounds = nb.bounds();
                 crx_draw_stats ds;
                 st = draw_views(lane.ctx, inst.data(), U, inst.data(), U, xf.data(), targets.data(), V, 0, lane.stream,
                                 &ds, ex);
@@ -805,6 +848,20 @@ crx_status crx_server_start(crx_server* s) {
         hipError_t e = hipMalloc(&s->cache, (size_t)s->numSlots * slot);
         if (e != hipSuccess) { s->cache = nullptr; return fail(CRX_OUT_OF_MEMORY, std::string("node cache: ") + hipGetErrorString(e)); }
     }
+    for (size_t i = 0; i < s->nodes.size(); i++) {
+        Node& n = s->nodes[i];
+        // nodes cut from one grid often share an index buffer
+        const Node* before = i ? &s->nodes[i - 1] : nullptr;
+        if (before && before->hidx == n.hidx && before->numTriangles == n.numTriangles) n.rowTris = before->rowTris;
+        else if (n.hidx) n.rowTris = detect_row_triangles(n.hidx, std::min<uint64_t>(n.numTriangles, kRowWindow));
+        DrawItem it{};
+        s->slotUnits = std::max(s->slotUnits, node_units(n, &it));
+    }
+    if (s->numSlots && s->slotUnits &&
+        hipMalloc((void**)&s->boxes, (size_t)s->numSlots * s->slotUnits * sizeof(UnitBox)) != hipSuccess) {
+        (void)hipGetLastError();
+        s->boxes = nullptr;     // draws without boxes draw the same
+    }
     s->slotNode.assign(s->numSlots, -1);
     s->slotReaders.assign(s->numSlots, 0u);
     hipError_t e = hipMalloc(&s->frames, s->cfg.frame_bytes);
@@ -882,6 +939,7 @@ crx_status crx_server_destroy(crx_server* s) {
     for (Node& n : s->nodes)
         if (n.ready) (void)hipEventDestroy(n.ready);
     if (s->cache) (void)hipFree(s->cache);
+    if (s->boxes) (void)hipFree(s->boxes);
     if (s->frames) (void)hipFree(s->frames);
     delete s;
     return CRX_OK;

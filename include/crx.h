@@ -232,7 +232,8 @@ typedef struct crx_draw_stats {
     uint32_t stage1_kernel;        /* the stage-1 kernel the draw ran: 0 = k_stage1 (lanes take
                                       triangles a block apart) or, for draws of few triangles per
                                       pixel, k_stage1_coarse, 1 = k_stage1_views (several views),
-                                      2 = k_stage1_pairs (consecutive pairs, tuning.stage1_layout) */
+                                      2 = k_stage1_pairs (consecutive pairs, tuning.stage1_layout;
+                                      also several views of meshes that hold unit boxes) */
 } crx_draw_stats;
 
 typedef struct crx_context crx_context;
