@@ -498,6 +498,26 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
         D.g1 = D.listed ? (uint32_t)ctx->numCUs * 10u : grid_for(ctx, sched.wavesPerCU, D.block / 64);
         if (D.g1 > D.batches) D.g1 = (uint32_t)D.batches;
     }
+    if (D.instanceBoxes && numViews == 1) {
+        // A batch's instances are shared by several workgroups.  Shares of
+        // about four instances take no box tests and spread the large
+        // triangles of near instances over the chip (600 nodes of 24 meshes:
+        // 720 us per frame in one share, 406 in four, 393 in six, 409 in
+        // eight, where the vertices are fetched too often).  A draw of so many instances
+        // that such shares are past number keeps long ones, which the box
+        // tests thin out, as few as give the chip two rounds of waves (3000
+        // instances of a 1 M-triangle mesh: 1247 us per frame in one share,
+        // 1280 in two, 1474 in eight).
+        uint64_t tris = 0;
+        for (uint32_t k = 0; k < D.numItems; k++) tris += list[k].numTriangles;
+        const uint64_t waves = std::max<uint64_t>(1, (uint64_t)D.g1 * (D.block / 64));
+        const uint64_t resident = (uint64_t)ctx->numCUs * 28u;
+        const uint64_t mean = tris ? (D.tris + tris - 1) / tris : 1;      // instances of a triangle
+        const uint64_t fine = std::min<uint64_t>((mean + 3) / 4, 1024);
+        D.instanceShares = (uint32_t)(waves * fine <= 16 * resident
+                                          ? fine
+                                          : std::min<uint64_t>(fine, std::max<uint64_t>(1, 2 * resident / waves)));
+    }
     D.g1 = (D.g1 + 7u) & ~7u;   // the stage-1 XCD split assumes a multiple of 8 workgroups
     D.g2 = grid_for(ctx, tu.stage2_waves_per_cu, 4);
     D.g3 = grid_for(ctx, tu.stage3_waves_per_cu, 4);
@@ -568,7 +588,7 @@ hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& D, const RasterParam
     else if (D.numViews == 1 && !viewsKernel && D.coarse)
         e = launch_stage1_coarse(P, D.g1, D.pu16, stream);
     else if (D.numViews == 1 && !viewsKernel)
-        e = launch_stage1(P, D.block, D.trisPerLane, D.g1, D.pu16, D.instanceBoxes, stream);
+        e = launch_stage1(P, D.block, D.trisPerLane, D.g1, D.pu16, D.instanceBoxes, D.instanceShares, stream);
     else e = launch_stage1_views(P, D.block, D.trisPerLane, D.g1, D.pu16, stream);
     if (e != hipSuccess) return e;
     record(ctx, T_S2, stream);

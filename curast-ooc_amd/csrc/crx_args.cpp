@@ -214,7 +214,7 @@ crx_status crx_raster_stage1(crx_context* ctx, const crx_raster_args* a, uint32_
     CRX_TRY(args_buffer(ctx, L.bytes, s, &dev));
     const ArgsLaunch r = args_launch(ctx, a, instanced, pu16, numItems, dev, L);
     CRX_HIP(build_records(a, instanced, pu16, numItems, r.P.batchShift, dev, L, s));
-    CRX_HIP(launch_stage1(r.P, ctx->tuning.stage1_block, r.perLane, r.g1, pu16, instanced, s));
+    CRX_HIP(launch_stage1(r.P, ctx->tuning.stage1_block, r.perLane, r.g1, pu16, instanced, 1u, s));
     return args_done(ctx, s);
 }
 
@@ -267,7 +267,7 @@ crx_status crx_raster_visbuffer_noalloc(crx_context* ctx, const crx_raster_args*
     // transforms and view, which stage 1's records include
     const ArgsLaunch r = args_launch(ctx, a, instanced, pu16, numItems, dev, L);
     CRX_HIP(build_records(a, instanced, pu16, numItems, r.P.batchShift, dev, L, s));
-    CRX_HIP(launch_stage1(r.P, ctx->tuning.stage1_block, r.perLane, r.g1, pu16, instanced, s));
+    CRX_HIP(launch_stage1(r.P, ctx->tuning.stage1_block, r.perLane, r.g1, pu16, instanced, 1u, s));
     CRX_HIP(launch_stage2(r.P, r.g2, s));
     CRX_HIP(launch_stage3(r.P, r.g3, s));
     return CRX_OK;

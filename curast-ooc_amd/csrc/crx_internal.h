@@ -24,8 +24,9 @@ hipError_t launch_store_view(const ViewParams& v, ViewParams* dst, hipStream_t s
 // pu16: the draw's meshes are IX_PU16-compressed
 // instanceBoxes: the draw repeats meshes over many instances (wave boxes
 // let groups of triangles skip instances that cull them all as tiny)
+// shares: workgroups that share the instances of a batch (instanceBoxes; at least 1)
 hipError_t launch_stage1(const RasterParams& P, uint32_t block, uint32_t trisPerLane, uint32_t grid, bool pu16,
-                         bool instanceBoxes, hipStream_t stream);
+                         bool instanceBoxes, uint32_t shares, hipStream_t stream);
 // Draws of few triangles per pixel, block 256: lane groups of 2^P.splitShift
 // per triangle (P.batchShift = 8 - P.splitShift), LDS raster tiles.
 hipError_t launch_stage1_coarse(const RasterParams& P, uint32_t grid, bool pu16, hipStream_t stream);

@@ -1052,6 +1052,25 @@ struct WaveBox {
     float M;   // max |coordinate| over the box
 };
 
+// The same box as its centre and half extents, these widened by 2^-18*M (the
+// roundings of the centre and the extent are below 2u*M, u = 2^-24).
+struct CenterBox {
+    f3 c, e;
+};
+
+// (of a wave-uniform box: the values stay in scalar registers)
+__device__ __forceinline__ float uni_f(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+}
+
+__device__ __forceinline__ CenterBox center_box(const WaveBox& B) {
+    const float w = 0x1p-18f * B.M;
+    return CenterBox{f3{uni_f(0.5f * B.lo.x + 0.5f * B.hi.x), uni_f(0.5f * B.lo.y + 0.5f * B.hi.y),
+                        uni_f(0.5f * B.lo.z + 0.5f * B.hi.z)},
+                     f3{uni_f(0.5f * B.hi.x - 0.5f * B.lo.x + w), uni_f(0.5f * B.hi.y - 0.5f * B.lo.y + w),
+                        uni_f(0.5f * B.hi.z - 0.5f * B.lo.z + w)}};
+}
+
 // Culling planes of one view for one instance, from its world-to-view
 // transform m: g(p) = a.p + b, with g > 0 meaning "outside".
 //   x+ : fa*x_view + z_view    (RN(fa*x/d) > 1,  d = -z_view)
@@ -1102,16 +1121,18 @@ __device__ __forceinline__ float box_max(const float* a, const WaveBox& B) {
             fmaxf(a[2] * B.lo.z, a[2] * B.hi.z)) + a[3];
 }
 
-// Range of the computed view coordinate of row r of m over the box.  With
-// S = (|m_r0| + |m_r1| + |m_r2|) * M + |m_r3|, the per-triangle code's
-// xform_row and this bound are each within 8u*S of the exact affine value
-// (u = 2^-24: three products and three sums); the widening is 2^-18*S, 8x more.
-__device__ __forceinline__ void row_range(const float* m, int r, const WaveBox& B, float& lo, float& hi) {
-    const float a[4] = {m[r], m[4 + r], m[8 + r], m[12 + r]};
-    const float S = ((fabsf(a[0]) + fabsf(a[1])) + fabsf(a[2])) * B.M + fabsf(a[3]);
-    const float e = S * 0x1p-18f;
-    lo = box_min(a, B) - e;
-    hi = box_max(a, B) + e;
+// Range of the computed view coordinate of row r of m over the box: the row
+// at the centre, plus and minus the row's magnitudes over the half extents.
+// With S = (|m_r0| + |m_r1| + |m_r2|) * M + |m_r3|, the per-triangle code's
+// xform_row and this bound are each within 8u*S of the exact affine value (u =
+// 2^-24); the extents and the last term widen it by 2^-18*S, 8x more.
+__device__ __forceinline__ void row_range(const float* m, int r, const CenterBox& B, float& lo, float& hi) {
+    const float a0 = m[r], a1 = m[4 + r], a2 = m[8 + r], a3 = m[12 + r];
+    const float c = __builtin_fmaf(a2, B.c.z, __builtin_fmaf(a1, B.c.y, __builtin_fmaf(a0, B.c.x, a3)));
+    const float e = __builtin_fmaf(fabsf(a2), B.e.z, __builtin_fmaf(fabsf(a1), B.e.y,
+                                   __builtin_fmaf(fabsf(a0), B.e.x, fabsf(a3) * 0x1p-18f)));
+    lo = c - e;
+    hi = c + e;
 }
 
 // True when every computed screen coordinate of one axis lies strictly
@@ -1139,7 +1160,7 @@ __device__ __forceinline__ bool axis_between_samples(float qlo, float qhi, float
 // strictly between the same two sample centres k and k + 1 with 0 <= k and
 // k + 1 <= size - 1, so the clamp changes nothing and each triangle's box
 // holds no sample.
-__device__ __forceinline__ bool wave_tiny_culled(const float* m, const ViewParams& V, const WaveBox& B) {
+__device__ __forceinline__ bool wave_tiny_culled(const float* m, const ViewParams& V, const CenterBox& B) {
     float xlo, xhi, ylo, yhi, zlo, zhi;
     row_range(m, 2, B, zlo, zhi);
     const float dlo = -zhi, dhi = -zlo;                 // depth = -view z
@@ -1223,6 +1244,64 @@ __device__ __forceinline__ bool wave_box(const f3& A, const f3& B, const f3& C, 
     return !unbounded;
 }
 
+// Screen position of a vertex within a small margin of the exact one, for
+// the filters of k_stage1_pairs and k_stage1: the exact view rows, and the quotients as
+// products with v_rcp_f32.  With |ndc| <= 2 the quotient is within 2^-21 of
+// the IEEE one and the screen coordinate, with the roundings of both screen
+// transforms, within 2^-20.7 * size; the filter's margin is 2^-19 * max(W, H).
+struct FilterView {
+    float gx, gy, cx, cy;    // half a size times the focal factor, and the screen centre
+    float W, H, margin;
+};
+
+__device__ __forceinline__ FilterView filter_view(const ViewParams& V) {
+    const float hx = 0.5f * V.Wf, hy = 0.5f * V.Hf;
+    return FilterView{V.fa * hx, V.f * hy, hx - 0.5f, hy - 0.5f, V.Wf, V.Hf, fmaxf(V.Wf, V.Hf) * 0x1p-19f};
+}
+
+struct FV {
+    float x, y, d;
+};
+
+__device__ __forceinline__ FV filter_vertex(const FilterView& F, const float* m, f3 p) {
+    FV v;
+    v.d = -xform_row(m, 2, p);
+    const float r = __builtin_amdgcn_rcpf(v.d);
+    v.x = __builtin_fmaf(xform_row(m, 0, p), F.gx * r, F.cx);
+    v.y = __builtin_fmaf(xform_row(m, 1, p), F.gy * r, F.cy);
+    return v;
+}
+
+// True only when the exact code (stage1_core) neither draws nor queues the
+// triangle.  All behind the camera: culled.  Otherwise, with every depth in
+// [2^-100, 2^100], when its box lies off one side by a sample or more (all
+// quotients beyond 1 in magnitude by more than the margin: the frustum test
+// culls it), or strictly between two neighbouring sample rows or columns k - 1
+// and k.  For 0 < k < size the tiny-triangle test culls that; for k = size
+// too, as the clamp brings the box's upper end to size - 1 only; for k = 0
+// the clamped box holds no sample (size_x or size_y is 0); beyond those the
+// frustum test has it.  Coordinates further off have larger errors, but
+// which of the cases they fall in does not depend on those.  A NaN or
+// infinite coordinate is NaN or infinite in both.
+__device__ __forceinline__ bool filter_culls(const FilterView& F, bool inside, const FV& a, const FV& b, const FV& c) {
+    const float lox = fminf(a.x, fminf(b.x, c.x)), hix = fmaxf(a.x, fmaxf(b.x, c.x));
+    const float loy = fminf(a.y, fminf(b.y, c.y)), hiy = fmaxf(a.y, fmaxf(b.y, c.y));
+    const bool tiny = (hix + F.margin < ceilf(lox - F.margin)) | (hiy + F.margin < ceilf(loy - F.margin));
+    if (inside) return tiny;   // wave-uniform: the depths are positive and no side is crossed
+    const float dmin = fminf(a.d, fminf(b.d, c.d)), dmax = fmaxf(a.d, fmaxf(b.d, c.d));
+    const bool safe = (dmin >= 0x1p-100f) & (dmax <= 0x1p100f) & (a.d == a.d) & (b.d == b.d) & (c.d == c.d);
+    const bool behind = (a.d <= 0.0f) & (b.d <= 0.0f) & (c.d <= 0.0f);
+    return behind | (safe & (tiny | (lox > F.W) | (hix < -1.0f) | (loy > F.H) | (hiy < -1.0f)));
+}
+
+// Rank of the lane among the lanes of a mask.
+__device__ __forceinline__ uint32_t mask_rank(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// Instances of a workgroup's share up to which k_stage1 draws them all, without box tests.
+constexpr uint32_t kBoxTestInstances = 8;
+
 // Lanes per group of the per-group instance lists of k_stage1 (8 or 16).
 constexpr int kBoxGroup = 16;
 
@@ -1260,14 +1339,17 @@ __device__ __forceinline__ void group_boxes(const f3& A, const f3& B, const f3& 
 // Stage 1 (stage1_drawSmallTriangles, triangles_visbuffer.cu:274-384): every
 // lane draws its K triangles into the single view, once per instance of the
 // item.
-// The variant that draws meshes over many instances with one triangle per
-// lane (the per-draw schedule for such draws) is held to 72 VGPRs, seven
-// waves per SIMD: its instance-list steps hide latency with waves, and the
-// few spilled registers cost less (1.56 -> 1.44 ms of stage 1 for 3000
-// instances of a 1M-triangle mesh); other variants keep the default, where a
-// VGPR limit spills far more.
+// Meshes over many instances are bound by VALU issue.  3000 instances of a
+// 1 M-triangle mesh take 3.45 M steps of 52 live lanes, of which 2.9 M
+// (triangle, instance) pairs hold a sample: the steps filter (1.46 -> 1.06 ms
+// of stage 1, 1218 M -> 752 M VALU instructions), and the boxes are held as
+// centre and extents, in scalar registers (752 M -> 676 M, 1.01 ms).  The
+// variant with one triangle per lane (the per-draw schedule for such draws) is
+// held to five waves per SIMD, which leaves it the 96 VGPRs it needs without
+// scratch (600 nodes: 390 us per frame at seven waves with spills, 372 at
+// five).
 template <int BLOCK, int K, bool PU16, bool BOXES>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && K == 1 ? 7 : 1))) void k_stage1(RasterParams P) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && K == 1 ? 5 : 1))) void k_stage1(RasterParams P) {
     // the view's record in device memory (a frame graph rewrites it between
     // launches; the kernel arguments stay as captured)
     const ViewParams V0 = kconst(P.views)[0];
@@ -1278,56 +1360,78 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && 
         words = pu16Words[threadIdx.x / kWave];
     }
     uint32_t* queue = nullptr;
+    uint2* left = nullptr;
     if constexpr (BOXES) {
         __shared__ uint32_t instQueue[BLOCK / kWave][2 * kWave];
+        __shared__ uint2 leftQueue[BLOCK / kWave][2 * kWave];
         queue = instQueue[threadIdx.x / kWave];
+        left = leftQueue[threadIdx.x / kWave];
     }
     s1_sweep<BLOCK, K, PU16>(P, words, [&](const S1Item& it, uint32_t base, const f3 (&A)[K], const f3 (&B)[K],
                                            const f3 (&C)[K]) __attribute__((always_inline)) {
+        // this workgroup's share of the item's instances (one of gridDim.y)
+        const uint32_t share = (it.instCount + gridDim.y - 1u) / gridDim.y;
+        const uint32_t jBegin = min(it.instCount, blockIdx.y * share);
+        const uint32_t jEnd = min(it.instCount, jBegin + share);
         if (BOXES && it.instCount >= kBoxInstances) {
-            // A mesh drawn over many instances.  Per wave group: 64 instances
-            // at a time, one per lane, are tested against the box of the
-            // wave's 64 triangles (wave_tiny_culled), and the instances it
-            // keeps are queued in LDS.  Each 64 queued instances are tested
-            // against the boxes of the wave's lane groups of kBoxGroup
-            // triangles, which leaves each group its own list of instances
-            // to draw.  Every step then draws, in each group, the next
-            // instance of that group's list, with the transform read from the
-            // lane that tested it: the wave takes as many steps as its
-            // longest list holds instances.
+            // A mesh drawn over many instances.  Per wave: 64 instances at a
+            // time, one per lane, are tested against the box of the wave's 64
+            // triangles (wave_tiny_culled), and the instances it keeps are
+            // queued in LDS.  Each 64 queued instances are tested against the
+            // boxes of the wave's lane groups of kBoxGroup triangles, which
+            // leaves each group its own list of instances to draw.  Every
+            // step then takes, in each group, the next instance of that
+            // group's list, with the transform read from the lane that tested
+            // it: the wave takes as many steps as its longest list holds
+            // instances.  A step only filters (filter_culls); the (triangle,
+            // instance) pairs it leaves are queued and drawn 64 at a time.
+            // A share of few instances is drawn without the box tests, which
+            // cost as much as the filter of about six instances.
             constexpr int NG = kWave / kBoxGroup;
             const uint32_t lane = threadIdx.x & (kWave - 1);
             const uint32_t grp = lane / kBoxGroup;
             const uint32_t cullOrder = item_cull_order(P, it.instCount);
             const auto xf = kglobal(V0.transforms) + it.instOffset;
+            const FilterView F = filter_view(V0);
+            const bool boxes = share > kBoxTestInstances;
+            if (jBegin >= jEnd) return;
             #pragma unroll
             for (int k = 0; k < K; k++) {
                 const uint32_t tri = base + k * BLOCK + threadIdx.x;
                 if (__ballot(tri < it.numTriangles) == 0ull) continue;
                 WaveBox wbox, gbox[NG];
-                bool gbounded[NG];
-                const bool wbounded = wave_box(A[k], B[k], C[k], wbox);
-                group_boxes<kBoxGroup>(A[k], B[k], C[k], gbox, gbounded);
-                uint32_t queued = 0;
-                for (uint32_t jb = 0;; jb += kWave) {
-                    const bool more = jb < it.instCount;
+                CenterBox wc{}, gc[NG] = {};
+                bool gbounded[NG] = {};
+                bool wbounded = false;
+                if (boxes) {
+                    wbounded = wave_box(A[k], B[k], C[k], wbox);
+                    group_boxes<kBoxGroup>(A[k], B[k], C[k], gbox, gbounded);
+                    wc = center_box(wbox);
+                    #pragma unroll
+                    for (int g = 0; g < NG; g++) gc[g] = center_box(gbox[g]);
+                }
+                uint32_t queued = 0, pairs = 0;
+                for (uint32_t jb = jBegin;; jb += kWave) {
+                    const bool more = jb < jEnd;
                     if (more) {
                         const uint32_t j = jb + lane;
-                        const auto Tj = xf + min(j, it.instCount - 1u);
-                        float mm[16];
-                        #pragma unroll
-                        for (int e = 0; e < 16; e++) mm[e] = Tj->m[e];
-                        const bool keep = j < it.instCount && !(wbounded && wave_tiny_culled(mm, V0, wbox));
+                        bool keep = j < jEnd;
+                        if (boxes) {
+                            const auto Tj = xf + min(j, jEnd - 1u);
+                            float mm[16];
+                            #pragma unroll
+                            for (int e = 0; e < 16; e++) mm[e] = Tj->m[e];
+                            keep = keep && !(wbounded && wave_tiny_culled(mm, V0, wc));
+                        }
                         const uint64_t kept = __ballot(keep);
-                        const uint32_t slot = __builtin_amdgcn_mbcnt_hi((uint32_t)(kept >> 32),
-                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0u));
-                        if (keep) queue[queued + slot] = j;   // queued < 64: slot < 128
+                        if (keep) queue[queued + mask_rank(kept)] = j;   // queued < 64: below 128
                         queued += (uint32_t)__popcll(kept);
                     }
-                    if (queued >= kWave || (!more && queued > 0u)) {
+                    // (past the last instance also to draw the pairs left over)
+                    if (queued >= kWave || (!more && (queued > 0u || pairs > 0u))) {
                         wave_sync();
                         const uint32_t n = min(queued, (uint32_t)kWave);
-                        const uint32_t qj = queue[min(lane, n - 1u)];
+                        const uint32_t qj = n ? queue[min(lane, n - 1u)] : jBegin;
                         const uint32_t rest = queue[kWave + lane];
                         wave_sync();
                         if (kWave + lane < queued) queue[lane] = rest;
@@ -1336,16 +1440,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && 
                         float mq[16];
                         #pragma unroll
                         for (int e = 0; e < 16; e++) mq[e] = Tq->m[e];
-                        const uint32_t fq = Tq->flip;
                         uint64_t q[NG];
                         #pragma unroll
                         for (int g = 0; g < NG; g++)
-                            q[g] = __ballot(lane < n && !(gbounded[g] && wave_tiny_culled(mq, V0, gbox[g])));
+                            q[g] = __ballot(lane < n && !(gbounded[g] && wave_tiny_culled(mq, V0, gc[g])));
                         for (;;) {
                             uint64_t any = 0ull;
                             #pragma unroll
                             for (int g = 0; g < NG; g++) any |= q[g];
-                            if (!any) break;
+                            const bool final = !more && queued == 0u;
+                            if (!any && !(final && pairs > 0u)) break;
                             uint32_t src = 0;
                             bool act = false;
                             #pragma unroll
@@ -1362,13 +1466,36 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && 
                             float m[16];
                             #pragma unroll
                             for (int e = 0; e < 16; e++) m[e] = __shfl(mq[e], (int)src);
-                            const uint32_t flip = (uint32_t)__shfl((int)fq, (int)src);
                             const uint32_t jj = (uint32_t)__shfl((int)qj, (int)src);
-                            if (act && tri < it.numTriangles) {
-                                const uint32_t inst = it.instOffset + jj;
-                                const uint64_t id = it.cumm + (uint64_t)tri + (uint64_t)(jj * it.numTriangles);
-                                stage1_triangle(P, V0, m, flip != 0u, A[k], B[k], C[k], id,
-                                                ((uint64_t)inst << 32) | (uint64_t)tri, cullOrder);
+                            const FV va = filter_vertex(F, m, A[k]), vb = filter_vertex(F, m, B[k]),
+                                     vc = filter_vertex(F, m, C[k]);
+                            const bool draw = act && tri < it.numTriangles && !filter_culls(F, false, va, vb, vc);
+                            const uint64_t drawn = __ballot(draw);
+                            if (draw) left[pairs + mask_rank(drawn)] = make_uint2(lane, jj);   // pairs < 64
+                            pairs += (uint32_t)__popcll(drawn);
+                            any = 0ull;
+                            #pragma unroll
+                            for (int g = 0; g < NG; g++) any |= q[g];
+                            const bool end = final && any == 0ull;
+                            while (pairs >= kWave || (end && pairs > 0u)) {
+                                const uint32_t np = min(pairs, (uint32_t)kWave);
+                                pairs -= np;
+                                wave_sync();
+                                const uint2 e = left[pairs + min(lane, np - 1u)];
+                                wave_sync();
+                                const int from = (int)e.x;
+                                const f3 a{__shfl(A[k].x, from), __shfl(A[k].y, from), __shfl(A[k].z, from)};
+                                const f3 b{__shfl(B[k].x, from), __shfl(B[k].y, from), __shfl(B[k].z, from)};
+                                const f3 c{__shfl(C[k].x, from), __shfl(C[k].y, from), __shfl(C[k].z, from)};
+                                const uint32_t t = tri - lane + e.x, inst = it.instOffset + e.y;
+                                const auto Te = xf + e.y;
+                                float me[16];
+                                #pragma unroll
+                                for (int i = 0; i < 16; i++) me[i] = Te->m[i];
+                                const uint64_t id = it.cumm + (uint64_t)t + (uint64_t)(e.y * it.numTriangles);
+                                if (lane < np)
+                                    stage1_triangle(P, V0, me, Te->flip != 0u, a, b, c, id,
+                                                    ((uint64_t)inst << 32) | (uint64_t)t, cullOrder);
                             }
                         }
                     }
@@ -1377,7 +1504,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && 
             }
             return;
         }
-        for (uint32_t j = 0; j < it.instCount; j++) {
+        for (uint32_t j = jBegin; j < jEnd; j++) {
             const uint32_t inst = it.instOffset + j;
             const auto T = transforms + inst;
             float m[16];
@@ -2035,61 +2162,6 @@ __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* 
 }
 
 namespace {
-
-// Screen position of a vertex within a small margin of the exact one, for
-// the filter of k_stage1_pairs: the exact view rows, and the quotients as
-// products with v_rcp_f32.  With |ndc| <= 2 the quotient is within 2^-21 of
-// the IEEE one and the screen coordinate, with the roundings of both screen
-// transforms, within 2^-20.7 * size; the filter's margin is 2^-19 * max(W, H).
-struct FilterView {
-    float gx, gy, cx, cy;    // half a size times the focal factor, and the screen centre
-    float W, H, margin;
-};
-
-__device__ __forceinline__ FilterView filter_view(const ViewParams& V) {
-    const float hx = 0.5f * V.Wf, hy = 0.5f * V.Hf;
-    return FilterView{V.fa * hx, V.f * hy, hx - 0.5f, hy - 0.5f, V.Wf, V.Hf, fmaxf(V.Wf, V.Hf) * 0x1p-19f};
-}
-
-struct FV {
-    float x, y, d;
-};
-
-__device__ __forceinline__ FV filter_vertex(const FilterView& F, const float* m, f3 p) {
-    FV v;
-    v.d = -xform_row(m, 2, p);
-    const float r = __builtin_amdgcn_rcpf(v.d);
-    v.x = __builtin_fmaf(xform_row(m, 0, p), F.gx * r, F.cx);
-    v.y = __builtin_fmaf(xform_row(m, 1, p), F.gy * r, F.cy);
-    return v;
-}
-
-// True only when the exact code (stage1_core) neither draws nor queues the
-// triangle.  All behind the camera: culled.  Otherwise, with every depth in
-// [2^-100, 2^100], when its box lies off one side by a sample or more (all
-// quotients beyond 1 in magnitude by more than the margin: the frustum test
-// culls it), or strictly between two neighbouring sample rows or columns k - 1
-// and k.  For 0 < k < size the tiny-triangle test culls that; for k = size
-// too, as the clamp brings the box's upper end to size - 1 only; for k = 0
-// the clamped box holds no sample (size_x or size_y is 0); beyond those the
-// frustum test has it.  Coordinates further off have larger errors, but
-// which of the cases they fall in does not depend on those.  A NaN or
-// infinite coordinate is NaN or infinite in both.
-__device__ __forceinline__ bool filter_culls(const FilterView& F, bool inside, const FV& a, const FV& b, const FV& c) {
-    const float lox = fminf(a.x, fminf(b.x, c.x)), hix = fmaxf(a.x, fmaxf(b.x, c.x));
-    const float loy = fminf(a.y, fminf(b.y, c.y)), hiy = fmaxf(a.y, fmaxf(b.y, c.y));
-    const bool tiny = (hix + F.margin < ceilf(lox - F.margin)) | (hiy + F.margin < ceilf(loy - F.margin));
-    if (inside) return tiny;   // wave-uniform: the depths are positive and no side is crossed
-    const float dmin = fminf(a.d, fminf(b.d, c.d)), dmax = fmaxf(a.d, fmaxf(b.d, c.d));
-    const bool safe = (dmin >= 0x1p-100f) & (dmax <= 0x1p100f) & (a.d == a.d) & (b.d == b.d) & (c.d == c.d);
-    const bool behind = (a.d <= 0.0f) & (b.d <= 0.0f) & (c.d <= 0.0f);
-    return behind | (safe & (tiny | (lox > F.W) | (hix < -1.0f) | (loy > F.H) | (hiy < -1.0f)));
-}
-
-// Rank of the lane among the lanes of a mask.
-__device__ __forceinline__ uint32_t mask_rank(uint64_t mask) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
 
 // The triangles that the filter left, per wave: fewer than 64 from earlier
 // batches and up to 128 (of half a batch, 64) more.
@@ -3545,21 +3617,21 @@ hipError_t launch_plan(const crx_cmesh* list, uint32_t numItems, const crx_cmesh
 namespace {
 
 template <int BLOCK, int K, bool PU16>
-hipError_t launch_s1(const RasterParams& P, uint32_t grid, bool views, bool boxes, hipStream_t stream) {
-    if (views) hipLaunchKernelGGL((k_stage1_views<BLOCK, K, PU16>), dim3(grid), dim3(BLOCK), 0, stream, P);
-    else if (boxes) hipLaunchKernelGGL((k_stage1<BLOCK, K, PU16, true>), dim3(grid), dim3(BLOCK), 0, stream, P);
-    else hipLaunchKernelGGL((k_stage1<BLOCK, K, PU16, false>), dim3(grid), dim3(BLOCK), 0, stream, P);
+hipError_t launch_s1(const RasterParams& P, dim3 grid, bool views, bool boxes, hipStream_t stream) {
+    if (views) hipLaunchKernelGGL((k_stage1_views<BLOCK, K, PU16>), grid, dim3(BLOCK), 0, stream, P);
+    else if (boxes) hipLaunchKernelGGL((k_stage1<BLOCK, K, PU16, true>), grid, dim3(BLOCK), 0, stream, P);
+    else hipLaunchKernelGGL((k_stage1<BLOCK, K, PU16, false>), grid, dim3(BLOCK), 0, stream, P);
     return hipGetLastError();
 }
 
 template <int BLOCK, int K>
-hipError_t launch_s1_fmt(const RasterParams& P, uint32_t grid, bool pu16, bool views, bool boxes, hipStream_t stream) {
+hipError_t launch_s1_fmt(const RasterParams& P, dim3 grid, bool pu16, bool views, bool boxes, hipStream_t stream) {
     return pu16 ? launch_s1<BLOCK, K, true>(P, grid, views, boxes, stream)
                 : launch_s1<BLOCK, K, false>(P, grid, views, boxes, stream);
 }
 
 template <int BLOCK>
-hipError_t launch_s1_k(const RasterParams& P, uint32_t k, uint32_t grid, bool pu16, bool views, bool boxes,
+hipError_t launch_s1_k(const RasterParams& P, uint32_t k, dim3 grid, bool pu16, bool views, bool boxes,
                        hipStream_t stream) {
     switch (k) {
         case 1: return launch_s1_fmt<BLOCK, 1>(P, grid, pu16, views, boxes, stream);
@@ -3569,7 +3641,7 @@ hipError_t launch_s1_k(const RasterParams& P, uint32_t k, uint32_t grid, bool pu
     }
 }
 
-hipError_t launch_s1_any(const RasterParams& P, uint32_t block, uint32_t k, uint32_t grid, bool pu16, bool views,
+hipError_t launch_s1_any(const RasterParams& P, uint32_t block, uint32_t k, dim3 grid, bool pu16, bool views,
                          bool boxes, hipStream_t stream) {
     switch (block) {
         case 128: return launch_s1_k<128>(P, k, grid, pu16, views, boxes, stream);
@@ -3582,8 +3654,8 @@ hipError_t launch_s1_any(const RasterParams& P, uint32_t block, uint32_t k, uint
 }  // namespace
 
 hipError_t launch_stage1(const RasterParams& P, uint32_t block, uint32_t trisPerLane, uint32_t grid, bool pu16,
-                         bool instanceBoxes, hipStream_t stream) {
-    return launch_s1_any(P, block, trisPerLane, grid, pu16, false, instanceBoxes, stream);
+                         bool instanceBoxes, uint32_t shares, hipStream_t stream) {
+    return launch_s1_any(P, block, trisPerLane, dim3(grid, shares), pu16, false, instanceBoxes, stream);
 }
 
 hipError_t launch_stage1_coarse(const RasterParams& P, uint32_t grid, bool pu16, hipStream_t stream) {
@@ -3627,7 +3699,7 @@ hipError_t launch_unit_bounds(const DrawItem& item, bool pu16, uint32_t numUnits
 
 hipError_t launch_stage1_views(const RasterParams& P, uint32_t block, uint32_t trisPerLane, uint32_t grid, bool pu16,
                                hipStream_t stream) {
-    return launch_s1_any(P, block, trisPerLane, grid, pu16, true, false, stream);
+    return launch_s1_any(P, block, trisPerLane, dim3(grid), pu16, true, false, stream);
 }
 
 hipError_t launch_resolve_views(const ResolveParams* views, uint32_t numViews, uint32_t numBlocks, bool full,
