@@ -1370,9 +1370,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BOXES && 
     s1_sweep<BLOCK, K, PU16>(P, words, [&](const S1Item& it, uint32_t base, const f3 (&A)[K], const f3 (&B)[K],
                                            const f3 (&C)[K]) __attribute__((always_inline)) {
         // this workgroup's share of the item's instances (one of gridDim.y)
-        const uint32_t share = (it.instCount + gridDim.y - 1u) / gridDim.y;
-        const uint32_t jBegin = min(it.instCount, blockIdx.y * share);
-        const uint32_t jEnd = min(it.instCount, jBegin + share);
+        uint32_t share = it.instCount, jBegin = 0u, jEnd = it.instCount;
+        if constexpr (BOXES) {
+            share = (it.instCount + gridDim.y - 1u) / gridDim.y;
+            jBegin = min(it.instCount, blockIdx.y * share);
+            jEnd = min(it.instCount, jBegin + share);
+        }
         if (BOXES && it.instCount >= kBoxInstances) {
             // A mesh drawn over many instances.  Per wave: 64 instances at a
             // time, one per lane, are tested against the box of the wave's 64
@@ -1722,16 +1725,13 @@ __global__ __launch_bounds__(256) void k_stage1_coarse(RasterParams P) {
 // those share two vertices: B = (A.a, A.c, n) for a grid cut along one
 // diagonal, B = (A.a, n, A.b) for the other (a lat-long sphere).  When every
 // lane of a wave holds one of these two patterns (the same one), the wave
-// gathers 4 vertices instead of 6 and computes each vertex's depth and view
-// y row once for both triangles (stage1_core<true>: the same operations, so
-// the same bits); other waves draw both triangles separately.  The six
-// indices are read with one 16- and one 8-byte buffer load.  Each wave
+// gathers 4 vertices instead of 6 and projects each once for the filter of
+// both triangles.  The six indices are read with one 16- and one 8-byte buffer load.  Each wave
 // claims units of unitRows consecutive rows of a 128-triangle strip (see
 // DrawItem::rowTris) and draws them row after row, so for a grid the vertex
 // row two neighbouring rows share is still in its XCD's L2 when the second
 // row reads it; claims are dynamic, which keeps the view-dependent cost of
-// the units balanced.  Only the order and the sharing of identical values
-// differ from k_stage1.
+// the units balanced.
 // ---------------------------------------------------------------------------
 
 constexpr uint32_t kPairNone = 0, kPairGrid = 1, kPairFan = 2;
@@ -2244,6 +2244,24 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(PU16 || V
             for (int e = 0; e < 16; e++) m[e] = T->m[e];
             const bool flip = T->flip != 0u;
             const bool skip = VIEWS && T->skip != 0u;   // dropped from this view
+            if constexpr (!LISTED) {
+                // Most units of a mesh walked whole lie off the view: a wave
+                // whose pairs are all above or all below it (the exact
+                // frustum test of the y axis, which stage1_core runs first)
+                // needs neither x nor the quotients (400 M-triangle terrain
+                // walked whole: 1515 us per frame, 1556 without this test,
+                // 1542 with the exact code on every triangle).
+                if (pat != kPairNone) {
+                    bool above = true, below = true;
+                    #pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float d = -xform_row(m, 2, S[v]), p = V.f * xform_row(m, 1, S[v]), t = d * 0x1p-24f;
+                        above = above & (d >= 0x1p-102f) & (p - d > t);
+                        below = below & (d >= 0x1p-102f) & (p + d < -t);
+                    }
+                    if (__ballot(!(above | below)) == 0ull && !(last && queued > 0u)) continue;
+                }
+            }
             const FV v0 = filter_vertex(F, m, S[0]), v1 = filter_vertex(F, m, S[1]), v2 = filter_vertex(F, m, S[2]),
                      v3 = filter_vertex(F, m, S[3]);
             const bool keepA = count > 0u && !skip && !filter_culls(F, LISTED && inside, v0, v1, v2);
