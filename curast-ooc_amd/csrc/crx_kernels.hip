@@ -1896,8 +1896,12 @@ __device__ __forceinline__ RunBatch part_first(const RunLayout& L, uint64_t part
         const uint32_t rows = kUnitRows >> partShift;
         b.row = uni(b.row + ((uint32_t)part & 0xFFu) * rows);
         b.rowEnd = uni(min(b.rowEnd, b.row + rows));
-        b.row = uni(min(b.row, L.rows - 1u));   // (a part past the last row is empty: run_bounds of its one batch)
-        if (b.row >= b.rowEnd) b.strip = 0xFFFFFFFFu;
+    }
+    if (LISTED && b.row >= b.rowEnd) {
+        // past the item's last row (the last unit's last parts, and the units
+        // that pad a strip): one batch without triangles
+        b.strip = 0xFFFFFFFFu;
+        b.row = b.rowEnd = uni(L.rows - 1u);
     }
     return b;
 }
