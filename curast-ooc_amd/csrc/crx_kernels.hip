@@ -1897,12 +1897,7 @@ __device__ __forceinline__ RunBatch part_first(const RunLayout& L, uint64_t part
         b.row = uni(b.row + ((uint32_t)part & 0xFFu) * rows);
         b.rowEnd = uni(min(b.rowEnd, b.row + rows));
     }
-    if (LISTED && b.row >= b.rowEnd) {
-        // past the item's last row (the last unit's last parts, and the units
-        // that pad a strip): one batch without triangles
-        b.strip = 0xFFFFFFFFu;
-        b.row = b.rowEnd = uni(L.rows - 1u);
-    }
+    // (a part past the item's last row: one batch, which run_bounds finds empty)
     return b;
 }
 
