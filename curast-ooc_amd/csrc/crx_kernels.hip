@@ -1263,6 +1263,14 @@ struct FV {
     float x, y, d;
 };
 
+// Minimum and maximum of three, NaN when one of them is.
+__device__ __forceinline__ float min3_nan(float a, float b, float c) {
+    return __builtin_elementwise_minimum(a, __builtin_elementwise_minimum(b, c));
+}
+__device__ __forceinline__ float max3_nan(float a, float b, float c) {
+    return __builtin_elementwise_maximum(a, __builtin_elementwise_maximum(b, c));
+}
+
 __device__ __forceinline__ FV filter_vertex(const FilterView& F, const float* m, f3 p) {
     FV v;
     v.d = -xform_row(m, 2, p);
@@ -1282,16 +1290,19 @@ __device__ __forceinline__ FV filter_vertex(const FilterView& F, const float* m,
 // the clamped box holds no sample (size_x or size_y is 0); beyond those the
 // frustum test has it.  Coordinates further off have larger errors, but
 // which of the cases they fall in does not depend on those.  A NaN or
-// infinite coordinate is NaN or infinite in both.
+// infinite coordinate is NaN or infinite in both; the minima and maxima pass a
+// NaN on (v_minimum3_f32), so that a coordinate or depth that is NaN in one
+// vertex only (inf - inf in one view row) decides nothing here.
 __device__ __forceinline__ bool filter_culls(const FilterView& F, bool inside, const FV& a, const FV& b, const FV& c) {
-    const float lox = fminf(a.x, fminf(b.x, c.x)), hix = fmaxf(a.x, fmaxf(b.x, c.x));
-    const float loy = fminf(a.y, fminf(b.y, c.y)), hiy = fmaxf(a.y, fmaxf(b.y, c.y));
-    const bool tiny = (hix + F.margin < ceilf(lox - F.margin)) | (hiy + F.margin < ceilf(loy - F.margin));
-    if (inside) return tiny;   // wave-uniform: the depths are positive and no side is crossed
-    const float dmin = fminf(a.d, fminf(b.d, c.d)), dmax = fmaxf(a.d, fmaxf(b.d, c.d));
-    const bool safe = (dmin >= 0x1p-100f) & (dmax <= 0x1p100f) & (a.d == a.d) & (b.d == b.d) & (c.d == c.d);
-    const bool behind = (a.d <= 0.0f) & (b.d <= 0.0f) & (c.d <= 0.0f);
-    return behind | (safe & (tiny | (lox > F.W) | (hix < -1.0f) | (loy > F.H) | (hiy < -1.0f)));
+    const float lox = min3_nan(a.x, b.x, c.x), hix = max3_nan(a.x, b.x, c.x);
+    const float loy = min3_nan(a.y, b.y, c.y), hiy = max3_nan(a.y, b.y, c.y);
+    // (bitwise: no branches between the comparisons)
+    const int tiny = (int)(hix + F.margin < ceilf(lox - F.margin)) | (int)(hiy + F.margin < ceilf(loy - F.margin));
+    if (inside) return tiny != 0;   // wave-uniform: the depths are positive and no side is crossed
+    const float dmin = min3_nan(a.d, b.d, c.d), dmax = max3_nan(a.d, b.d, c.d);
+    const int off = (int)(lox > F.W) | (int)(hix < -1.0f) | (int)(loy > F.H) | (int)(hiy < -1.0f);
+    const int safe = (int)(dmin >= 0x1p-100f) & (int)(dmax <= 0x1p100f);
+    return ((int)(dmax <= 0.0f) | (safe & (tiny | off))) != 0;
 }
 
 // Rank of the lane among the lanes of a mask.
