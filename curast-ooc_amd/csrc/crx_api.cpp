@@ -1048,6 +1048,8 @@ uint32_t scene_lists(crx_scene* scene, const crx_view* views, uint32_t numViews,
         scene->nodeOf.resize(n);
         scene->uniqueBounds.resize(n);
         scene->instanceBounds.resize(n);
+        scene->uniqueMesh.resize(n);
+        scene->instanceMesh.resize(n);
         uint64_t sum = 0;
         uint32_t u = 0;
         for (uint32_t i = 0; i < n; i++) {
@@ -1080,10 +1082,12 @@ uint32_t scene_lists(crx_scene* scene, const crx_view* views, uint32_t numViews,
             scene->nodeOf[i] = kept[i];
             sum += cm.numTriangles;
             scene->instances[i] = cm;
-            scene->instanceBounds[i] = nd.mesh->shared ? nullptr : nd.mesh->bounds;
+            scene->instanceBounds[i] = *nd.mesh->handedOut ? nullptr : nd.mesh->bounds;
+            scene->instanceMesh[i] = nd.mesh;
             if (u == 0 || scene->unique[u - 1].address != cm.address || !settings.instanced) {
                 scene->unique[u] = cm;
                 scene->uniqueBounds[u] = scene->instanceBounds[i];
+                scene->uniqueMesh[u] = nd.mesh;
                 u++;
             }
             scene->unique[u - 1].instances.count++;
@@ -1900,10 +1904,7 @@ crx_status crx_mesh_buffers(const crx_mesh* mesh, const float** d_positions, con
     if (d_indices) *d_indices = mesh->indices;
     if (d_colors) *d_colors = mesh->colors;
     // whoever holds the addresses may write there: the boxes no longer count
-    if (!mesh->shared) {
-        mesh->shared = true;
-        mesh->ctx->attrEpoch++;
-    }
+    if (!mesh->handedOut->exchange(true)) mesh->ctx->attrEpoch++;
     return CRX_OK;
 }
 

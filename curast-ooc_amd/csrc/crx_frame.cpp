@@ -6,13 +6,18 @@
 // the three stages (every stage reads the views' records from device memory,
 // so new cameras only need new staging contents), a copy
 // of the counters back to page-locked memory and the resolve.  Launching the
-// frame is one hipGraphLaunch; new cameras rewrite the staging buffers.  The
+// frame is one hipGraphLaunch; new cameras rewrite the staging buffers.  A
+// launch itself reads neither the scene nor the tuning: it only takes the
+// unit boxes of meshes whose geometry was handed out from the draw items.  The
 // clear and the counter reset are kernels: the graph records no memset node.
 #include "crx.h"
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -32,7 +37,13 @@ struct crx_frame {
 
     DrawPlan plan;
     size_t nodes = 0;                 // scene node count at creation
-    uint64_t attrEpoch = 0;           // the context's attrEpoch the records were written at
+    // draw items in the staging image that hold unit boxes, and whether
+    // crx_mesh_buffers has handed their mesh's geometry out since
+    struct BoxedItem {
+        uint32_t item;
+        std::shared_ptr<std::atomic<bool>> handedOut;
+    };
+    std::vector<BoxedItem> boxed;
     DeviceBuffer drawMeta, resolveMeta, clearMeta, nontrivial, huge, unitList;
     uint32_t ntCap = 0, hugeCap = 0;
     uint32_t* ctr = nullptr;          // device counters
@@ -74,7 +85,6 @@ crx_status frame_fill(crx_frame* F, bool write) {
     CRX_TRY(plan_draw(F->ctx, sc->unique.data(), u, sc->instances.data(), n, sc->transforms.data(), targets.data(),
                       F->numViews, F->settings.instanced, F->settings.frustum_culling ? sc->skip.data() : nullptr,
                       &D, false, false, bounds));
-    F->attrEpoch = F->ctx->attrEpoch;
     std::vector<char> rimage;
     size_t offViews = 0;
     uint32_t rblocks = 0;
@@ -109,6 +119,25 @@ crx_status frame_fill(crx_frame* F, bool write) {
     F->P.units = static_cast<uint64_t*>(F->unitList.ptr);
     if (!rimage.empty()) std::memcpy(F->stageResolve, rimage.data(), rimage.size());
     if (!cv.empty()) std::memcpy(F->stageClear, cv.data(), F->clearBytes);
+    const auto& meshes = F->settings.instanced ? sc->uniqueMesh : sc->instanceMesh;
+    F->boxed.clear();
+    for (uint32_t k = 0; k < D.numItems; k++)
+        if (D.items[k].bounds) F->boxed.push_back({k, meshes[k]->handedOut});
+    return CRX_OK;
+}
+
+// Takes the boxes of meshes whose geometry was handed out from the frame's
+// draw items: such an item draws every unit.
+crx_status frame_drop_boxes(crx_frame* F) {
+    if (std::none_of(F->boxed.begin(), F->boxed.end(), [](const auto& b) { return b.handedOut->load(); })) return CRX_OK;
+    if (F->launched) CRX_HIP(hipEventSynchronize(F->done));   // the graph reads the staging buffers
+    DrawItem* items = reinterpret_cast<DrawItem*>(static_cast<char*>(F->stageDraw) + F->plan.offItems);
+    const auto drop = [items](const crx_frame::BoxedItem& b) {
+        if (!b.handedOut->load()) return false;
+        items[b.item].bounds = nullptr;
+        return true;
+    };
+    F->boxed.erase(std::remove_if(F->boxed.begin(), F->boxed.end(), drop), F->boxed.end());
     return CRX_OK;
 }
 
@@ -249,11 +278,7 @@ crx_status crx_frame_set_views(crx_frame* F, const crx_view* views) {
 crx_status crx_frame_launch(crx_frame* F, void* stream) {
     if (!F) return fail(CRX_INVALID_ARG, "frame is NULL");
     CRX_HIP(hipSetDevice(F->ctx->device));
-    if (F->plan.listed && F->attrEpoch != F->ctx->attrEpoch) {
-        // a mesh may have lost its boxes (crx_mesh_buffers): write the records again
-        if (F->launched) CRX_HIP(hipEventSynchronize(F->done));
-        CRX_TRY(frame_fill(F, true));
-    }
+    CRX_TRY(frame_drop_boxes(F));
     CRX_HIP(hipGraphLaunch(F->exec, as_stream(stream)));
     CRX_HIP(hipEventRecord(F->done, as_stream(stream)));
     F->launched = true;

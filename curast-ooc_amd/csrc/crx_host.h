@@ -7,7 +7,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <functional>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -241,10 +243,11 @@ struct crx_mesh {
     crx_vec3 compressionFactor{};
     uint32_t rowTris = 0;             // triangles per row of a mesh stored in rows (0 = none found)
     // Boxes of the mesh's units in the default walk (plan_draw's pair layout),
-    // made with the mesh from the geometry it owns; null for small meshes and
-    // once crx_mesh_buffers has handed the geometry out.
+    // made with the mesh from the geometry it owns; null for small meshes.
+    // They no longer count once crx_mesh_buffers has handed the geometry out;
+    // recorded frames that hold them share that flag.
     crx::UnitBox* bounds = nullptr;
-    mutable bool shared = false;      // crx_mesh_buffers was called
+    std::shared_ptr<std::atomic<bool>> handedOut = std::make_shared<std::atomic<bool>>(false);
     // resolve-only vertex attributes, always owned by the mesh (crx_mesh_set_attributes)
     float* uvs = nullptr;             // 2 floats per vertex
     float* normals = nullptr;         // 3 floats per vertex
@@ -262,6 +265,7 @@ struct crx_scene {
     // frame-preparation scratch, kept across frames like the reference's statics
     std::vector<crx_cmesh> unique, instances;
     std::vector<const crx::UnitBox*> uniqueBounds, instanceBounds;   // crx_mesh::bounds of each entry
+    std::vector<const crx_mesh*> uniqueMesh, instanceMesh;           // and the meshes
     std::vector<crx_mat4> transforms;
     std::vector<uint64_t> prefix;
     std::vector<uint8_t> skip;        // [view][instance]: dropped by that view's node cull
