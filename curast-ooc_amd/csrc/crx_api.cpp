@@ -462,7 +462,10 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
         if (D.listed) it.bounds = bounds.boxes[k];
         D.batches += D.runs ? units : ((uint64_t)m.numTriangles + batchTris - 1) >> D.batchShift;
         D.tris += (uint64_t)m.numTriangles * (uint64_t)cnt;
-        if (D.listed && D.batches >= (1ull << 31)) return fail(CRX_INVALID_ARG, "too many triangle batches for one draw");
+        // (a list entry names a unit with 31 bits: such a draw takes the walk over all units)
+        if (D.listed && D.batches >= (1ull << 31))
+            return plan_draw(ctx, meshes, numMeshes, instances, numInstances, transforms, targets, numViews, instanced,
+                             skip, plan, instUnchanged, prefix, DrawBounds{});
         if (D.batches >= (1ull << 32)) return fail(CRX_INVALID_ARG, "too many triangle batches for one draw");
     }
     // instUnchanged: the list is the one the plan's records were built (and
