@@ -637,6 +637,12 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
     if (stats) stats->num_triangles = D.tris * numViews;
     if (D.batches == 0 && !ex.afterStages) return CRX_OK;
     CRX_HIP(hipSetDevice(ctx->device));
+    if (D.listed && ctx->unitList.reserve(D.batches * D.numViews * sizeof(uint64_t)) != CRX_OK) {
+        // without the memory for the list the same draw walks all units
+        (void)hipGetLastError();
+        CRX_TRY(plan_draw(ctx, meshes, numMeshes, instances, numInstances, transforms, targets, numViews, instanced,
+                          ex.skip, &D, sameLists, ex.prefix));
+    }
     CRX_TRY(wait_meta_free(ctx, stream));
 
     RasterParams P{};
@@ -682,7 +688,6 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
         return finish();
     }
     CRX_TRY(ensure_queues(ctx, ctx->tuning.max_nontrivial, ctx->tuning.max_huge));
-    if (D.listed) CRX_TRY(ctx->unitList.reserve(D.batches * D.numViews * sizeof(uint64_t)));
     P.units = static_cast<uint64_t*>(ctx->unitList.ptr);
 
     uint32_t redraws = 0;

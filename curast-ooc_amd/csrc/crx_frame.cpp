@@ -246,6 +246,11 @@ crx_status crx_frame_create(crx_context* ctx, crx_scene* scene, const crx_view* 
         if (st == CRX_OK) st = F->huge.reserve((size_t)F->hugeCap * sizeof(int4));
         if (st == CRX_OK && F->plan.listed) st = F->unitList.reserve(F->plan.batches * numViews * sizeof(uint64_t));
     }
+    if (st != CRX_OK) {
+        // no stream and no graph on a device without memory
+        crx_frame_destroy(F);
+        return st;
+    }
     hip(hipMalloc(&F->ctr, CTR_COUNT * sizeof(uint32_t)), "hipMalloc");
     hip(hipHostMalloc((void**)&F->ctrHost, CTR_COUNT * sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc");
     hip(hipHostMalloc(&F->stageDraw, std::max<size_t>(F->drawBytes, 256), hipHostMallocDefault), "hipHostMalloc");
