@@ -3720,6 +3720,7 @@ hipError_t launch_cull_units(const RasterParams& P, hipStream_t stream) {
 
 hipError_t launch_unit_bounds(const DrawItem& item, bool pu16, uint32_t numUnits, UnitBox* out, hipStream_t stream) {
     const uint32_t blocks = (numUnits + 3u) / 4u;
+    (void)hipGetLastError();   // an error that an earlier call left behind is not this launch's
     if (pu16) hipLaunchKernelGGL(k_unit_bounds<true>, dim3(blocks), dim3(256), 0, stream, item, numUnits, out);
     else hipLaunchKernelGGL(k_unit_bounds<false>, dim3(blocks), dim3(256), 0, stream, item, numUnits, out);
     return hipGetLastError();

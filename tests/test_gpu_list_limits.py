@@ -137,3 +137,12 @@ def test_more_units_than_entries_can_name(ctx, frame):
         fb.free()
         scene.close()
         mesh.close()
+
+
+def test_mesh_after_a_failed_allocation(ctx):
+    """An allocation that failed leaves its error behind in the runtime; a mesh made
+    next, whose boxes take a launch, is none the worse for it."""
+    with pytest.raises(crx.CrxError):
+        ctx.alloc(1 << 50)
+    mesh = _long_rows(ctx)
+    mesh.close()
