@@ -274,29 +274,37 @@ uint32_t row_hint_of(const void* indices) {
 uint32_t detect_row_triangles(const uint32_t* idx, uint64_t T) {
     const uint64_t W = std::min<uint64_t>(T, 1ull << 18);
     if (W < 1024) return 0;
-    const uint64_t t0 = T / 2 - W / 2;
-    std::unordered_map<uint32_t, uint64_t> first;
-    first.reserve(2 * W);
-    std::unordered_map<uint64_t, uint32_t> gaps;
-    std::unordered_map<uint32_t, uint8_t> done;
-    for (uint64_t t = t0; t < t0 + W; t++) {
-        for (int k = 0; k < 3; k++) {
-            const uint32_t v = idx[3 * t + k];
-            auto f = first.find(v);
-            if (f == first.end()) {
-                first.emplace(v, t);
-            } else if (t - f->second > 64 && !done[v]) {
-                done[v] = 1;
-                gaps[t - f->second]++;
-            }
+    const uint32_t* window = idx + 3 * (T / 2 - W / 2);
+    const auto range = std::minmax_element(window, window + 3 * W);
+    const uint32_t lo = *range.first;
+    const uint64_t span = (uint64_t)*range.second - lo + 1;
+    // per vertex: its first use in the window plus one, and in the top bit that its distance is counted
+    constexpr uint32_t kCounted = 0x80000000u;
+    std::vector<uint32_t> gaps(W, 0u);      // vertices by distance
+    uint64_t vertices = 0;
+    const auto use = [&](uint32_t& first, uint32_t t) {
+        if (first == 0u) {
+            first = t + 1u;
+            vertices++;
+        } else if (!(first & kCounted) && t + 1u - first > 64u) {
+            gaps[t + 1u - first]++;
+            first |= kCounted;
         }
+    };
+    // a window's vertices lie close together in most meshes: then an array
+    // holds them, at a twentieth of the time of a hash map
+    if (span <= 8 * W) {
+        std::vector<uint32_t> first(span, 0u);
+        for (uint32_t t = 0; t < W; t++)
+            for (int k = 0; k < 3; k++) use(first[window[3 * t + k] - lo], t);
+    } else {
+        std::unordered_map<uint32_t, uint32_t> first;
+        first.reserve(2 * W);
+        for (uint32_t t = 0; t < W; t++)
+            for (int k = 0; k < 3; k++) use(first[window[3 * t + k]], t);
     }
-    uint64_t best = 0;
-    uint32_t count = 0;
-    for (const auto& g : gaps)
-        if (g.second > count || (g.second == count && g.first < best)) { best = g.first; count = g.second; }
-    if (count * 4ull < first.size() || best > 0xFFFFFFFFull) return 0;
-    return (uint32_t)best & ~1u;
+    const uint64_t best = std::max_element(gaps.begin(), gaps.end()) - gaps.begin();   // the shortest of equals
+    return gaps[best] * 4ull < vertices ? 0u : (uint32_t)best & ~1u;
 }
 
 // Pair layout (batches of one wave's 128 triangles): units of stripRows rows

@@ -850,10 +850,13 @@ crx_status crx_server_start(crx_server* s) {
     }
     for (size_t i = 0; i < s->nodes.size(); i++) {
         Node& n = s->nodes[i];
-        // nodes cut from one grid often share an index buffer
+        // nodes cut from one grid have the same indices, in one buffer or in copies
         const Node* before = i ? &s->nodes[i - 1] : nullptr;
-        if (before && before->hidx == n.hidx && before->numTriangles == n.numTriangles) n.rowTris = before->rowTris;
-        else if (n.hidx) n.rowTris = detect_row_triangles(n.hidx, std::min<uint64_t>(n.numTriangles, kRowWindow));
+        const uint64_t window = std::min<uint64_t>(n.numTriangles, kRowWindow);
+        if (before && before->numTriangles == n.numTriangles && before->hidx && n.hidx &&
+            (before->hidx == n.hidx || std::memcmp(before->hidx, n.hidx, 12 * window) == 0))
+            n.rowTris = before->rowTris;
+        else if (n.hidx) n.rowTris = detect_row_triangles(n.hidx, window);
         DrawItem it{};
         s->slotUnits = std::max(s->slotUnits, node_units(n, &it));
     }

@@ -9,6 +9,9 @@ every eviction; a view of more nodes than the cache holds is drawn in groups.
 Every result equals the oracle's draw of the nodes the view sees (tolerance:
 none).
 """
+import ctypes
+import time
+
 import numpy as np
 import pytest
 
@@ -141,3 +144,41 @@ def test_results_equal_the_oracle(ctx, nodes, slots, batch, lanes):
         print(f"[server] slots {slots}: uploads {st.uploads} evictions {st.evictions} max batch {st.max_batch}", flush=True)
     finally:
         srv.close()
+
+
+def test_start_does_not_search_every_node(ctx):
+    """1000 nodes of 8192 triangles start about as fast with an index buffer each, of
+    the same or of alternating content, as with one for all: the search for a
+    node's row length may take 0.1 ms (hash maps over the window took 0.25 and more)."""
+    count = 1000
+    kinds = [_node(ctx, "rows", r, c, 0.0, 0.0, 1) for r, c in ((64, 64), (32, 128))]
+    words = 3 * 8192
+    copies = crx.PinnedBuffer(ctx, 4 * words * count)
+    idx = copies.array(np.uint32, words * count).reshape(count, words)
+    try:
+        nodes = [n for _, n in kinds]
+        took = {}
+        for name in ("shared", "copies", "alternating"):
+            for k in range(count):
+                nd = nodes[k % 2 if name == "alternating" else 0]
+                idx[k] = np.ctypeslib.as_array((ctypes.c_uint32 * words).from_address(nd["idx"]))
+            best = 1e9
+            for _ in range(4):
+                srv = crx.Server(ctx, crx.server_config(node_cache_bytes=16 << 20, frame_bytes=1 << 20,
+                                                        max_batch_views=4, lanes=1, resolve=0, prefetch=0))
+                for k in range(count):
+                    nd = nodes[k % 2 if name == "alternating" else 0]
+                    at = nd["idx"] if name == "shared" else copies.ptr + 4 * words * k
+                    srv.add_node(nd["pos"], nd["nv"], at, nd["nt"], nd["col"], nd["aabb"])
+                t0 = time.perf_counter()
+                srv.start()
+                best = min(best, time.perf_counter() - t0)
+                srv.close()
+            took[name] = best
+        print("[server] start of 1000 nodes:", {k: f"{1e3 * v:.1f} ms" for k, v in took.items()}, flush=True)
+        assert took["copies"] < took["shared"] + 1e-4 * count
+        assert took["alternating"] < took["shared"] + 1e-4 * count
+    finally:
+        copies.free()
+        for b, _ in kinds:
+            b.free()
