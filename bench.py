@@ -609,14 +609,15 @@ def main() -> int:
         ctx.close()
         return 0
 
-    draw_stats = None
     for _ in range(max(1, args.warmup)):
-        draw_stats = scene.render(v, fb, cb, settings)
+        scene.render(v, fb, cb, settings)
     ctx.synchronize()
-    # the stage-1 kernel the draw took (crx_draw_stats::stage1_kernel)
-    kernel = {0: ("k_stage1<256, 2, true, false>" if args.compressed else "k_stage1"), 1: "k_stage1_views",
-              2: "k_stage1_pairs<256, %s>" % ("true" if args.compressed else "false")}.get(
-        draw_stats.stage1_kernel, "k_stage1")
+    # the stage-1 kernel the draw took
+    route = ctx.stage1_launch().route
+    fmt = "true" if args.compressed else "false"
+    kernel = {crx.STAGE1_PLAIN: f"k_stage1<256, 2, {fmt}, false>" if args.compressed else "k_stage1",
+              crx.STAGE1_VIEWS: "k_stage1_views", crx.STAGE1_COARSE: f"k_stage1_coarse<{fmt}>"}.get(
+        route, f"k_stage1_pairs<256, {fmt}>")
 
     atomics = bench_atomics(ctx)
     log(f"[bench] atomicMin probe: {atomics}")
@@ -669,7 +670,7 @@ def main() -> int:
     if args.workload == "instances":
         algo = mesh_bytes + 64 * len(worlds)
     share = None
-    if args.workload == "heightfield" and draw_stats.stage1_kernel == 2:
+    if args.workload == "heightfield" and route == crx.STAGE1_LISTED:
         # the draw reads the units that the view may see: what it cannot do
         # without is the geometry inside the view
         share = seen_share(pos, view, proj)

@@ -168,6 +168,15 @@ class DrawStats(C.Structure):
                 ("num_huge", C.c_uint32), ("redraws", C.c_uint32), ("stage1_kernel", C.c_uint32)]
 
 
+# crx_stage1_route: the stage-1 kernel a draw took
+(STAGE1_NONE, STAGE1_PLAIN, STAGE1_VIEWS, STAGE1_PAIRS, STAGE1_COARSE, STAGE1_LISTED,
+ STAGE1_LISTED_VIEWS) = range(7)
+
+
+class Stage1Launch(C.Structure):
+    _fields_ = [("route", C.c_uint32), ("workgroups", C.c_uint32), ("shares", C.c_uint32), ("split", C.c_uint32)]
+
+
 class AutotuneResult(C.Structure):
     _fields_ = [("tuning", Tuning), ("start_ms", C.c_float), ("best_ms", C.c_float),
                 ("trials", C.c_uint32), ("reserved", C.c_uint32)]
@@ -248,6 +257,7 @@ _SIGS = {
     "crx_context_num_cus": (C.c_int, [_VP, C.POINTER(C.c_int)]),
     "crx_context_enable_timing": (C.c_int, [_VP, C.c_int]),
     "crx_context_timings": (C.c_int, [_VP, C.POINTER(Timings)]),
+    "crx_context_stage1_launch": (C.c_int, [_VP, C.POINTER(Stage1Launch)]),
     "crx_device_alloc": (C.c_int, [_VP, C.c_size_t, C.POINTER(_VP)]),
     "crx_device_free": (C.c_int, [_VP, _VP]),
     "crx_memcpy_htod": (C.c_int, [_VP, _VP, _VP, C.c_size_t, _VP]),
@@ -298,6 +308,7 @@ _SIGS = {
     "crx_server_release": (C.c_int, [_VP, C.c_uint64]),
     "crx_server_clock": (C.c_double, [_VP]),
     "crx_server_get_stats": (C.c_int, [_VP, C.POINTER(ServerStats)]),
+    "crx_server_stage1_launch": (C.c_int, [_VP, C.c_uint32, C.POINTER(Stage1Launch)]),
     "crx_server_view_nodes": (C.c_int, [_VP, C.POINTER(View), C.POINTER(C.c_uint32), C.c_uint32,
                                         C.POINTER(C.c_uint32)]),
     "crx_autotune": (C.c_int, [_VP, _VP, C.POINTER(View), C.c_uint32, C.POINTER(_VP), C.c_uint32, C.c_uint32,
@@ -483,6 +494,12 @@ class Context:
         t = Timings()
         _check(lib().crx_context_timings(self.handle, C.byref(t)))
         return t
+
+    def stage1_launch(self) -> Stage1Launch:
+        """How the last draw launched stage 1 (route: one of STAGE1_*)."""
+        out = Stage1Launch()
+        _check(lib().crx_context_stage1_launch(self.handle, C.byref(out)))
+        return out
 
     def alloc(self, nbytes: int) -> DeviceBuffer:
         b = DeviceBuffer(self, nbytes)
@@ -915,6 +932,12 @@ class Server:
         st = ServerStats()
         _check(lib().crx_server_get_stats(self.handle, C.byref(st)))
         return st
+
+    def stage1_launch(self, lane: int) -> Stage1Launch:
+        """The stage-1 launch of a lane's last batch, with no request in flight."""
+        out = Stage1Launch()
+        _check(lib().crx_server_stage1_launch(self.handle, lane, C.byref(out)))
+        return out
 
     def view_nodes(self, view: View) -> list[int]:
         n = C.c_uint32()

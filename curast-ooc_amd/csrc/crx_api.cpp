@@ -612,6 +612,26 @@ hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& D, const RasterParam
     return hipSuccess;
 }
 
+// The stage 1 that enqueue_stages launches for a plan.
+crx_stage1_launch stage1_launch(const DrawPlan& D) {
+    crx_stage1_launch L{};
+    if (D.batches == 0) return L;
+    L.workgroups = D.g1;
+    L.shares = L.split = 1u;
+    if (D.runs) {
+        L.route = !D.listed ? CRX_STAGE1_PAIRS : D.numViews > 1 ? CRX_STAGE1_LISTED_VIEWS : CRX_STAGE1_LISTED;
+    } else if (D.numViews > 1) {
+        L.route = CRX_STAGE1_VIEWS;
+    } else if (D.coarse) {
+        L.route = CRX_STAGE1_COARSE;
+        L.split = 1u << D.splitShift;
+    } else {
+        L.route = CRX_STAGE1_PLAIN;
+        L.shares = D.instanceShares;
+    }
+    return L;
+}
+
 // Instance records (and prefix) from which a draw that finds them already in
 // the metadata buffer copies the rest in two pieces rather than all in one.
 constexpr size_t kSplitUploadBytes = 64 * 1024;
@@ -643,6 +663,7 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
     CRX_TRY(plan_draw(ctx, meshes, numMeshes, instances, numInstances, transforms, targets, numViews, instanced,
                       ex.skip, &D, sameLists, ex.prefix, ex.bounds));
     if (stats) stats->num_triangles = D.tris * numViews;
+    ctx->stage1 = stage1_launch(D);
     if (D.batches == 0 && !ex.afterStages) return CRX_OK;
     CRX_HIP(hipSetDevice(ctx->device));
     if (D.listed && ctx->unitList.reserve(D.batches * D.numViews * sizeof(uint64_t)) != CRX_OK) {
@@ -650,6 +671,7 @@ crx_status draw_views(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMes
         (void)hipGetLastError();
         CRX_TRY(plan_draw(ctx, meshes, numMeshes, instances, numInstances, transforms, targets, numViews, instanced,
                           ex.skip, &D, sameLists, ex.prefix));
+        ctx->stage1 = stage1_launch(D);
     }
     CRX_TRY(wait_meta_free(ctx, stream));
 
@@ -1358,6 +1380,12 @@ crx_status crx_context_timings(crx_context* ctx, crx_timings* out) {
     out->stage3_ms = span(T_S3, T_S3_END);
     out->pipeline_ms = span(T_S1, T_S3_END);
     out->resolve_ms = span(T_RESOLVE, T_RESOLVE_END);
+    return CRX_OK;
+}
+
+crx_status crx_context_stage1_launch(const crx_context* ctx, crx_stage1_launch* out) {
+    if (!ctx || !out) return fail(CRX_INVALID_ARG, "NULL argument");
+    *out = ctx->stage1;
     return CRX_OK;
 }
 

@@ -216,6 +216,7 @@ struct crx_context {
     bool timing = false;
     hipEvent_t ev[crx::T_COUNT] = {};
     bool recorded[crx::T_COUNT] = {};
+    crx_stage1_launch stage1{};       // of the last draw
     uint64_t meshSeq = 0;
     uint64_t attrEpoch = 0;           // bumped by every crx_mesh_set_attributes (and mesh's loss of its boxes)
     // kernel-level entry points: the records buffer every crx_raster_stage*

@@ -1008,6 +1008,12 @@ crx_status crx_server_release(crx_server* s, uint64_t ticket) {
 
 double crx_server_clock(const crx_server* s) { return s ? s->now() : 0.0; }
 
+crx_status crx_server_stage1_launch(const crx_server* s, uint32_t lane, crx_stage1_launch* out) {
+    if (!s || !out) return fail(CRX_INVALID_ARG, "NULL argument");
+    if (!s->started || lane >= s->lanes.size()) return fail(CRX_INVALID_ARG, "the server has no such lane");
+    return crx_context_stage1_launch(s->lanes[lane].ctx, out);
+}
+
 crx_status crx_server_get_stats(const crx_server* s_, crx_server_stats* out) {
     if (!s_ || !out) return fail(CRX_INVALID_ARG, "NULL argument");
     crx_server* s = const_cast<crx_server*>(s_);

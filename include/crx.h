@@ -409,6 +409,28 @@ crx_status crx_context_enable_timing(crx_context* ctx, int enable);
 /* Synchronises on the recorded events and returns their durations. */
 crx_status crx_context_timings(crx_context* ctx, crx_timings* out);
 
+/* The stage-1 kernel that a draw took. */
+typedef enum crx_stage1_route {
+    CRX_STAGE1_NONE = 0,          /* nothing to draw */
+    CRX_STAGE1_PLAIN = 1,         /* k_stage1 */
+    CRX_STAGE1_VIEWS = 2,         /* k_stage1_views */
+    CRX_STAGE1_PAIRS = 3,         /* k_stage1_pairs over all units */
+    CRX_STAGE1_COARSE = 4,        /* k_stage1_coarse (few triangles per pixel) */
+    CRX_STAGE1_LISTED = 5,        /* k_stage1_pairs over the units that the view may see */
+    CRX_STAGE1_LISTED_VIEWS = 6   /* the same of several views */
+} crx_stage1_route;
+
+/* How the last draw of a context (crx_draw_*, crx_render*) launched stage 1.
+ * crx_draw_stats::stage1_kernel tells less: its 0 covers PLAIN and COARSE, its
+ * 2 PAIRS, LISTED and LISTED_VIEWS. */
+typedef struct crx_stage1_launch {
+    uint32_t route;        /* crx_stage1_route */
+    uint32_t workgroups;   /* in the grid, of each share */
+    uint32_t shares;       /* PLAIN: workgroups that share a batch's instances, else 1 */
+    uint32_t split;        /* COARSE: lanes that share a triangle, else 1 */
+} crx_stage1_launch;
+crx_status crx_context_stage1_launch(const crx_context* ctx, crx_stage1_launch* out);
+
 /* ------------------------------------------------------------------ */
 /* Device memory plumbing for C hosts (hipMalloc / hipMemcpy wrappers). */
 /* ------------------------------------------------------------------ */
@@ -745,6 +767,10 @@ typedef struct crx_server_stats {
 } crx_server_stats;
 
 crx_status crx_server_get_stats(const crx_server* server, crx_server_stats* out);
+
+/* The stage-1 launch of a lane's last batch (crx_context_stage1_launch), for a
+ * server with no request in flight. */
+crx_status crx_server_stage1_launch(const crx_server* server, uint32_t lane, crx_stage1_launch* out);
 
 /* Nodes a view draws (the node cull of that view), ascending ids; returns
  * their number in *count (at most `capacity` ids are written). */
