@@ -506,7 +506,7 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
     if (sched.wavesPerCU == 0 || D.coarse) {   // one workgroup per batch
         D.g1 = (uint32_t)std::min<uint64_t>(D.batches, 1ull << 31);
     } else {
-        D.g1 = D.listed ? (uint32_t)ctx->numCUs * 10u : grid_for(ctx, sched.wavesPerCU, D.block / 64);
+        D.g1 = grid_for(ctx, sched.wavesPerCU, D.block / 64);
         if (D.g1 > D.batches) D.g1 = (uint32_t)D.batches;
     }
     if (D.instanceBoxes && numViews == 1) {

@@ -126,3 +126,25 @@ def test_nothing_to_draw(ctx):
     assert ctx.stage1_launch().route == crx.STAGE1_NONE
     scene.close()
     fb.free()
+
+
+def test_grid_of_a_listed_draw(ctx, large):
+    """stage1_waves_per_cu sets the grid of a listed draw of one float view as it does
+    any other's; several views take 64 waves per CU."""
+    for waves in (8, 20, 32, 64):
+        got = _draw(ctx, [(large, None)], [(320, 200)], stage1_waves_per_cu=waves)
+        assert got.route == crx.STAGE1_LISTED
+        assert got.workgroups == min(ctx.num_cus * waves // 4, (_units(large) + 7) // 8 * 8)
+    got = _draw(ctx, [(large, None)], [(320, 200)], stage1_waves_per_cu=0)         # one workgroup per unit
+    assert got.workgroups == (_units(large) + 7) // 8 * 8
+    for waves in (8, 32):
+        got = _draw(ctx, [(large, None)], [(320, 200)] * 2, stage1_waves_per_cu=waves)
+        assert got.route == crx.STAGE1_LISTED_VIEWS
+        assert got.workgroups == min(ctx.num_cus * 16, (_units(large) + 7) // 8 * 8)
+
+
+def _units(mesh):
+    """Units of the default walk: strips of 128 triangles times groups of 8 rows, rounded up to 8."""
+    row = mesh.row_triangles()
+    rows = (mesh.num_triangles + row - 1) // row
+    return (row + 127) // 128 * (((rows + 7) // 8 + 7) // 8 * 8)
