@@ -1078,8 +1078,11 @@ uint32_t scene_lists(crx_scene* scene, const crx_view* views, uint32_t numViews,
     const int instancedFlag = settings.instanced ? 1 : 0;
     // the per-node records depend on the node set, the instancing switch and
     // the kept nodes only: a frame that changes none of them keeps them
+    // (the epoch is read before the meshes' flags: geometry handed out
+    // meanwhile, from another thread, is seen by the next frame at the latest)
+    const uint64_t epoch = scene->ctx->attrEpoch;
     if (scene->listsKey == 0 || scene->listsVersion != scene->version || scene->listsInstanced != instancedFlag ||
-        scene->listsAttrEpoch != scene->ctx->attrEpoch || scene->listsKept != kept) {
+        scene->listsAttrEpoch != epoch || scene->listsKept != kept) {
         scene->unique.resize(n);
         scene->instances.resize(n);
         scene->prefix.resize(n);
@@ -1132,7 +1135,7 @@ uint32_t scene_lists(crx_scene* scene, const crx_view* views, uint32_t numViews,
         }
         scene->unique.resize(u);
         scene->listsVersion = scene->version;
-        scene->listsAttrEpoch = scene->ctx->attrEpoch;
+        scene->listsAttrEpoch = epoch;
         scene->listsInstanced = instancedFlag;
         scene->listsKept.swap(kept);
         scene->listsKey = next_lists_key();

@@ -218,7 +218,9 @@ struct crx_context {
     bool recorded[crx::T_COUNT] = {};
     crx_stage1_launch stage1{};       // of the last draw
     uint64_t meshSeq = 0;
-    uint64_t attrEpoch = 0;           // bumped by every crx_mesh_set_attributes (and mesh's loss of its boxes)
+    // bumped by every crx_mesh_set_attributes, and when a mesh's geometry is
+    // handed out (crx_mesh_buffers may run beside a draw)
+    std::atomic<uint64_t> attrEpoch{0};
     // kernel-level entry points: the records buffer every crx_raster_stage*
     // call rebuilds its records in, and the event after the last call's
     // launches (a call on another stream waits for it)

@@ -6,7 +6,9 @@ each rule's line: few triangles per pixel and the lanes that share a triangle
 there, meshes with unit boxes, several views, the tuning's knobs, and meshes
 drawn over many instances.
 """
-import numpy as np
+import threading
+import time
+
 import pytest
 
 import crx
@@ -103,6 +105,37 @@ def test_handed_out_geometry(ctx):
     assert _draw(ctx, [(mesh, None)], [(320, 200)]).route == crx.STAGE1_PLAIN
     assert _draw(ctx, [(mesh, None)], [(320, 200)] * 2).route == crx.STAGE1_VIEWS
     mesh.close()
+
+
+def test_geometry_handed_out_beside_draws(ctx):
+    """Another thread hands meshes out while a scene of them is drawn: once it is
+    done, the next draw takes no boxes."""
+    meshes = [crx.Mesh(ctx, *wl.heightfield_mesh(726, amplitude=9.0, scale=90.0)) for _ in range(6)]
+    scene = crx.Scene(ctx)
+    for m in meshes:
+        scene.add(m)
+    view = crx.make_view(crx.look_at((360.0, 200.0, -100.0), (360.0, 0.0, 300.0)), wl.projection(320, 200), 320, 200)
+    fb = ctx.alloc(8 * 320 * 200)
+    settings = crx.render_settings(resolve=0)
+
+    def hand_out():
+        for m in meshes:
+            time.sleep(0.002)
+            m.buffers()
+
+    scene.render(view, fb, None, settings)
+    assert ctx.stage1_launch().route == crx.STAGE1_LISTED
+    other = threading.Thread(target=hand_out)
+    other.start()
+    while other.is_alive():
+        scene.render(view, fb, None, settings)
+    other.join()
+    scene.render(view, fb, None, settings)
+    assert ctx.stage1_launch().route == crx.STAGE1_PLAIN
+    scene.close()
+    fb.free()
+    for m in meshes:
+        m.close()
 
 
 def test_many_instances(ctx, large):
