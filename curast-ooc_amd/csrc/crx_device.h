@@ -28,7 +28,15 @@ struct UnitBox {
 // (crx_tuning::stage1_strip_rows), at 128 triangles (one wave) per row.
 constexpr uint32_t kUnitRows = 8;
 
-// Triangles from which a mesh gets unit boxes and a draw uses them.
+// Triangles from which a mesh gets unit boxes and a draw uses them.  The list
+// costs a launch of 5 us.  Stage 1 at 640 x 360 of terrains of 1.05, 2.1, 4.2
+// and 8.4 M triangles, k_stage1 against the listed pair kernel: seen whole 16,
+// 24, 38 and 61 us against 23, 30, 39 and 54, from their edge 16, 24, 41 and 55
+// against 23, 30, 40 and 47, from close up 34, 40, 45 and 48 against 49, 63, 54
+// and 50.  Eight views of mixed sizes, whole frames at 0.13, 0.26, 0.53, 1.05 and
+// 2.1 M: 253, 296, 324, 331 and 352 us with k_stage1_views against 274, 321, 323,
+// 326 and 342.  So the line is where several views gain; one view gains from 4 M
+// on, and between the two it loses 2 to 23 us.
 constexpr uint64_t kListMinTris = 1u << 20;
 
 // Most entries (units times views) of a draw's unit list: 256 MB of list.
