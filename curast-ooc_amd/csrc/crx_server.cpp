@@ -860,16 +860,17 @@ crx_status crx_server_start(crx_server* s) {
         DrawItem it{};
         s->slotUnits = std::max(s->slotUnits, node_units(n, &it));
     }
-    if (s->numSlots && s->slotUnits &&
-        hipMalloc((void**)&s->boxes, (size_t)s->numSlots * s->slotUnits * sizeof(UnitBox)) != hipSuccess) {
-        (void)hipGetLastError();
-        s->boxes = nullptr;     // draws without boxes draw the same
-    }
     s->slotNode.assign(s->numSlots, -1);
     s->slotReaders.assign(s->numSlots, 0u);
     hipError_t e = hipMalloc(&s->frames, s->cfg.frame_bytes);
     if (e != hipSuccess) { s->frames = nullptr; return fail(CRX_OUT_OF_MEMORY, std::string("frame arena: ") + hipGetErrorString(e)); }
     s->arena.init(s->cfg.frame_bytes);
+    // (last: the boxes take no memory that the start cannot do without)
+    if (s->numSlots && s->slotUnits &&
+        hipMalloc((void**)&s->boxes, (size_t)s->numSlots * s->slotUnits * sizeof(UnitBox)) != hipSuccess) {
+        (void)hipGetLastError();
+        s->boxes = nullptr;     // draws without boxes draw the same
+    }
     CRX_HIP(hipStreamCreateWithFlags(&s->upload, hipStreamNonBlocking));
     {
         std::lock_guard<std::mutex> lk(s->cacheMu);
