@@ -514,8 +514,8 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
         // about four instances take no box tests and spread the large
         // triangles of near instances over the chip (600 nodes of 24 meshes:
         // 720 us per frame in one share, 406 in four, 393 in six, 409 in
-        // eight, where the vertices are fetched too often).  A draw of so many instances
-        // that such shares are past number keeps long ones, which the box
+        // eight, where the vertices are fetched too often).  A draw of so many
+        // instances that such shares are past number keeps long ones, which the box
         // tests thin out, as few as give the chip two rounds of waves (3000
         // instances of a 1 M-triangle mesh: 1247 us per frame in one share,
         // 1280 in two, 1474 in eight).
@@ -591,12 +591,10 @@ hipError_t enqueue_stages(crx_context* ctx, const DrawPlan& D, const RasterParam
         if (e != hipSuccess) return e;
     }
     record(ctx, T_S1, stream);
-    if (!viewsKernel && D.runs)
-    {
+    if (!viewsKernel && D.runs) {
         if (D.listed) e = launch_cull_units(P, stream);
         if (e == hipSuccess) e = launch_stage1_pairs(P, D.block, D.g1, D.pu16, D.listed, stream);
-    }
-    else if (D.numViews == 1 && !viewsKernel && D.coarse)
+    } else if (D.numViews == 1 && !viewsKernel && D.coarse)
         e = launch_stage1_coarse(P, D.g1, D.pu16, stream);
     else if (D.numViews == 1 && !viewsKernel)
         e = launch_stage1(P, D.block, D.trisPerLane, D.g1, D.pu16, D.instanceBoxes, D.instanceShares, stream);

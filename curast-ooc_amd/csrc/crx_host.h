@@ -128,7 +128,7 @@ struct DrawPlan {
     uint32_t block = 256, trisPerLane = 1, batchShift = 8, g1 = 0, g2 = 0, g3 = 0;
     bool instanceBoxes = false;   // some item loops over >= 4 instances
     uint32_t instanceShares = 1;  // workgroups that share a batch's instances (k_stage1)
-    bool runs = false;            // k_stage1_runs (items carry the run layout; batches counts its units)
+    bool runs = false;            // k_stage1_pairs (items carry the pair layout; batches counts its units)
     bool listed = false;          // runs over the units k_cull_units lists (some item has boxes)
     bool coarse = false;          // k_stage1_coarse (few triangles per pixel)
     uint32_t splitShift = 0;      // its lanes per triangle (log2)

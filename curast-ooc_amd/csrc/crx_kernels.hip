@@ -1206,8 +1206,8 @@ __device__ __forceinline__ bool view_inside(const ViewCull& c, const WaveBox& B)
     const float mz = (c.slopeZ * B.M + c.cnstZ) * 0x1p-16f + 0x1p-90f;
     const float mx = (c.slopeX * B.M + c.cnstX) * 0x1p-16f + 0x1p-90f;
     const float my = (c.slopeY * B.M + c.cnstY) * 0x1p-16f + 0x1p-90f;
-    return box_max(c.z, B) < -mz && box_min(c.z, B) > -0x1p99f && mz < 0x1p99f && box_max(c.px, B) < -mx && box_max(c.nx, B) < -mx && box_max(c.py, B) < -my &&
-           box_max(c.ny, B) < -my;
+    return box_max(c.z, B) < -mz && box_min(c.z, B) > -0x1p99f && mz < 0x1p99f && box_max(c.px, B) < -mx &&
+           box_max(c.nx, B) < -mx && box_max(c.py, B) < -my && box_max(c.ny, B) < -my;
 }
 
 __device__ __forceinline__ ViewCull lane_view_cull(const RasterParams& P, uint32_t view, uint32_t inst) {
@@ -1245,8 +1245,8 @@ __device__ __forceinline__ bool wave_box(const f3& A, const f3& B, const f3& C, 
 }
 
 // Screen position of a vertex within a small margin of the exact one, for
-// the filters of k_stage1_pairs and k_stage1: the exact view rows, and the quotients as
-// products with v_rcp_f32.  With |ndc| <= 2 the quotient is within 2^-21 of
+// the filters of k_stage1_pairs and k_stage1: the exact view rows, and the
+// quotients as products with v_rcp_f32.  With |ndc| <= 2 the quotient is within 2^-21 of
 // the IEEE one and the screen coordinate, with the roundings of both screen
 // transforms, within 2^-20.7 * size; the filter's margin is 2^-19 * max(W, H).
 struct FilterView {
@@ -1740,12 +1740,12 @@ __global__ __launch_bounds__(256) void k_stage1_coarse(RasterParams P) {
 // diagonal, B = (A.a, n, A.b) for the other (a lat-long sphere).  When every
 // lane of a wave holds one of these two patterns (the same one), the wave
 // gathers 4 vertices instead of 6 and projects each once for the filter of
-// both triangles.  The six indices are read with one 16- and one 8-byte buffer load.  Each wave
-// claims units of unitRows consecutive rows of a 128-triangle strip (see
-// DrawItem::rowTris) and draws them row after row, so for a grid the vertex
-// row two neighbouring rows share is still in its XCD's L2 when the second
-// row reads it; claims are dynamic, which keeps the view-dependent cost of
-// the units balanced.
+// both triangles.  The six indices are read with one 16- and one 8-byte buffer
+// load.  Each wave takes units of unitRows consecutive rows of a 128-triangle
+// strip (see DrawItem::rowTris) and draws them row after row, so for a grid the
+// vertex row two neighbouring rows share is still in its XCD's L2 when the
+// second row reads it; whole units are claimed as the waves get to them, which
+// keeps their view-dependent cost balanced (UnitSource).
 // ---------------------------------------------------------------------------
 
 constexpr uint32_t kPairNone = 0, kPairGrid = 1, kPairFan = 2;
@@ -1755,10 +1755,10 @@ struct RunLayout {
     uint32_t rowTris, unitRows, unitSegs, unitCols, rows, firstUnit;
 };
 
-// A batch of the unit walk: unit (absolute), its strip, current row, the
-// batch's column in the strip and the unit's row end (wave-uniform scalars).
+// A batch of the unit walk: the unit's strip, the current row, the batch's
+// column in the strip and the unit's row end (wave-uniform scalars).
 struct RunBatch {
-    uint32_t unit, strip, row, col, rowEnd;
+    uint32_t strip, row, col, rowEnd;
     uint32_t inside;    // the unit lies inside the view (kUnitInside or 0)
     uint32_t view;      // listed: the view to draw it into
     uint32_t row0;      // squares: the unit's first row (`row` then counts its squares)
@@ -1825,7 +1825,6 @@ __device__ __forceinline__ RunBatch run_first(const RunLayout& L, uint32_t u) {
     b.inside = 0u;
     b.view = 0u;
     b.row0 = 0u;
-    b.unit = uni(u);
     b.strip = s;
     b.col = 0u;
     b.row = uni(g * L.unitRows);
@@ -2083,11 +2082,11 @@ __device__ __forceinline__ uint32_t pair_vertices(const S1Item& it, uint32_t bas
 
 // The batch walk of k_stage1_pairs, software-pipelined two deep like
 // s1_sweep: while batch i is drawn, the gathers of batch i+1 and the index
-// loads of batch i+2 are in flight.  Units (strip, group of rows) are dealt
-// to the workgroups by P.order as s1_range deals batches; a workgroup walks
-// its unit's rows in turn.  body(it, t, count, S, pattern, inside,
-// view, last) draws one batch, lane by lane `count` triangles from t; `last` marks the last one of a pass over an item, or
-// before another view's.
+// loads of batch i+2 are in flight.  Each wave takes units (strip, group of
+// rows), or parts of listed units, from its UnitSource and walks their rows in
+// turn.  body(it, t, count, S, pattern, inside, view, last) draws one batch,
+// lane by lane `count` triangles from t; `last` marks the last one of a pass
+// over an item, or before another view's.
 template <bool PU16, bool LISTED, bool SQUARE, typename Body>
 __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* words, Body&& body) {
     const uint32_t numUnits = P.batchCount ? *kconst(P.batchCount) : P.numBatches;
@@ -2127,12 +2126,12 @@ __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* 
         uint32_t n0, n1;
         uint32_t base0, end0, base1, end1, base2, end2;
         const RunBatch b0 = part_first<LISTED, SQUARE>(L, part, U.partShift);
-        bounds( b0, base0, end0);
+        bounds(b0, base0, end0);
         uint32_t I[6], J[6];
         pair_indices<PU16, SQUARE>(it, L.rowTris, base0, end0, lane, I);
         uint32_t more1;
         RunBatch b1 = run_next<LISTED, SQUARE>(L, U, iend, b0, more1, pending);
-        bounds( b1, base1, end1);
+        bounds(b1, base1, end1);
         pair_indices<PU16, SQUARE>(it, L.rowTris, base1, end1, lane, J);
         f3 S[6];
         (void)lane_tris<SQUARE>(it, L.rowTris, base0, end0, lane, n0);
@@ -2144,7 +2143,7 @@ __device__ __forceinline__ void s1_pairs_sweep(const RasterParams& P, uint32_t* 
             const uint32_t patN = pair_vertices<PU16>(it, base1, end1, lane, n1, words, J, Sn);
             uint32_t more2 = 0u;
             const RunBatch b2 = more1 ? run_next<LISTED, SQUARE>(L, U, iend, b1, more2, pending) : b1;
-            bounds( b2, base2, end2);
+            bounds(b2, base2, end2);
             pair_indices<PU16, SQUARE>(it, L.rowTris, base2, end2, lane, J);
             if constexpr (PU16) {
                 #pragma unroll
@@ -2407,9 +2406,8 @@ __global__ __launch_bounds__(256) void k_unit_bounds(DrawItem it, uint32_t numUn
 constexpr uint32_t kCullChunk = 1024;    // units per workgroup, one per lane
 
 // Lists the units of a draw that a view may see (workgroup c * views + v:
-// view v, chunk c; the views of a chunk follow each other, so that those that draw a
-// unit find it in the caches; view_may_see:
-// a unit is dropped only when every triangle in it is culled by its own exact
+// view v, chunk c; the views of a chunk follow each other, so that those that
+// draw a unit find it in the caches; view_may_see: a unit is dropped only when every triangle in it is culled by its own exact
 // tests), and marks those wholly inside it (kUnitInside; every instance's,
 // where the item has several).  One append per workgroup of 1024 units: the
 // returning atomics on the one counter take 6 ns each.  A terrain flown over

@@ -217,7 +217,11 @@ typedef struct crx_tuning {
                                      length detected from the index buffer by crx_mesh_create) is
                                      walked in units of stage1_strip_rows consecutive rows of a
                                      strip of stage1_strip_batches batches of 128 triangles, so the
-                                     vertex row two rows share is read once */
+                                     vertex row two rows share is read once.
+                                     Frames of at least 2^20 triangles in meshes that crx_mesh_create
+                                     (or a server) made draw only the units that the view may see, of
+                                     one view or several, float or IX_PU16, while the layout, the
+                                     strip and stage1_tris_per_lane are at their defaults */
     uint32_t stage1_strip_rows;   /* rows (or batches) per unit of layouts 1 and 2, 1..256 (default 8) */
     uint32_t stage1_strip_batches; /* layout 2: batches of 128 triangles side by side in a strip, 1..8
                                       (default 1); a unit's wave draws each row's batches left to right */
@@ -674,7 +678,10 @@ crx_status crx_frame_destroy(crx_frame* frame);
 typedef struct crx_server crx_server;
 
 typedef struct crx_server_config {
-    uint64_t node_cache_bytes;   /* device memory for resident node geometry (LRU cache of slots) */
+    uint64_t node_cache_bytes;   /* device memory for resident node geometry (LRU cache of slots); the
+                                    boxes of the nodes' units come on top, 32 bytes per 1024 triangles
+                                    (up to eight times that for nodes of a few long rows), and are
+                                    left out when they cannot be allocated */
     uint64_t frame_bytes;        /* device memory for in-flight result buffers: requests are
                                     admitted while their W*H*8 (x2 with resolve) bytes fit */
     uint32_t max_batch_views;    /* views per batched draw, 1..CRX_MAX_VIEWS */
