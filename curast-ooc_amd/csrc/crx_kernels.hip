@@ -1354,8 +1354,8 @@ __device__ __forceinline__ void group_boxes(const f3& A, const f3& B, const f3& 
 // 1 M-triangle mesh take 3.45 M steps of 52 live lanes, of which 2.9 M
 // (triangle, instance) pairs hold a sample: the steps filter (1.46 -> 1.06 ms
 // of stage 1, 1218 M -> 752 M VALU instructions), and the boxes are held as
-// centre and extents, in scalar registers (752 M -> 676 M, 1.01 ms).  The
-// variant with one triangle per lane (the per-draw schedule for such draws) is
+// centre and extents, in scalar registers (752 M -> 676 M, 1.01 ms; 662 M with
+// minima that pass a NaN on).  The variant with one triangle per lane (the per-draw schedule for such draws) is
 // held to five waves per SIMD, which leaves it the 96 VGPRs it needs without
 // scratch (600 nodes: 390 us per frame at seven waves with spills, 372 at
 // five).
@@ -2211,8 +2211,8 @@ struct LeftTris {
 // gathered in LDS and drawn 64 at a time by the exact code.  The positions are
 // kept with them: gathered again from memory they made the kernel fetch 600
 // MB in place of 520 and wait (143 us against 134).
-// Stage 1 of that terrain 195 -> 130 us (VALU instructions 112 M -> 50 M, 4.0
-// TB/s fetched), of the 400 M-triangle one's 1.5% in view 79 -> 62.
+// Stage 1 of that terrain 195 -> 139 us (VALU instructions 112 M -> 54 M, 3.7
+// TB/s fetched), of the 400 M-triangle one's 1.5% in view 79 -> 66.
 //
 // Several views: a unit is drawn once for every view that may see it, where
 // k_stage1_views tests every 64 triangles against every view.  Their triangles
@@ -2220,7 +2220,9 @@ struct LeftTris {
 // pairs, lane by lane, 71 M requests and 3.6 ms for 64 views, of which 2.3
 // remain when no sample is sent).  So a batch is a square of 8 rows of 8 pairs,
 // which fits the LDS tile of raster_wave: 43 M requests, 3.4 ms, against 4.3
-// of k_stage1_views (VALU instructions 2394 M -> 1914 M).  IX_PU16 streams are
+// of k_stage1_views (VALU instructions 2394 M -> 1910 M).  The waves that draw a
+// unit's views are not the same, so its geometry is fetched for each of them: 10
+// GB in place of 2.4, at 3 TB/s.  IX_PU16 streams are
 // cut per row, so they keep the rows and the lane's own atomics.
 template <int BLOCK, bool PU16, bool LISTED, bool VIEWS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(PU16 || VIEWS ? 1 : 5))) void k_stage1_pairs(RasterParams P) {
