@@ -616,8 +616,9 @@ def main() -> int:
     route = ctx.stage1_launch().route
     fmt = "true" if args.compressed else "false"
     kernel = {crx.STAGE1_PLAIN: f"k_stage1<256, 2, {fmt}, false>" if args.compressed else "k_stage1",
-              crx.STAGE1_VIEWS: "k_stage1_views", crx.STAGE1_COARSE: f"k_stage1_coarse<{fmt}>"}.get(
-        route, f"k_stage1_pairs<256, {fmt}>")
+              crx.STAGE1_VIEWS: "k_stage1_views", crx.STAGE1_COARSE: f"k_stage1_coarse<{fmt}>",
+              crx.STAGE1_LISTED: f"k_cull_units, k_stage1_pairs<256, {fmt}, true, false>"}.get(
+        route, f"k_stage1_pairs<256, {fmt}, false, false>")
 
     atomics = bench_atomics(ctx)
     log(f"[bench] atomicMin probe: {atomics}")

@@ -199,7 +199,10 @@ struct RasterParams {
     uint32_t* claims;        // k_stage1_pairs: the per-XCD unit counters (CTR_CLAIM of the counter block)
 };
 
-struct ResolveParams {
+// A copy of host records to the device whose length is no multiple of 16 bytes
+// takes a slower kernel (the resolve's records of 40 instances 3.8 us against
+// 2.3), so every record that ends one is a multiple of 16.
+struct alignas(16) ResolveParams {
     const InstanceRec* inst;
     const uint64_t* prefix;
     const uint64_t* fb;
@@ -226,6 +229,9 @@ struct ResolveParams {
 struct CounterSet {
     uint32_t* p[5];
 };
+
+static_assert(sizeof(ResolveParams) % 16 == 0 && sizeof(Transform) % 16 == 0 && CTR_COUNT * 4 % 16 == 0,
+              "records at the end of a copy");
 
 // One framebuffer of a multi-view clear.
 struct ClearView {
