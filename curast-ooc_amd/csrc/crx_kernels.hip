@@ -1905,10 +1905,10 @@ __device__ __forceinline__ RunBatch part_first(const RunLayout& L, uint64_t part
         b.rowEnd = uni(b.row + n);
         return b;
     }
-    if (LISTED && partShift > 0u) {
+    if constexpr (LISTED) {
         const uint32_t rows = kUnitRows >> partShift;
         b.row = uni(b.row + ((uint32_t)part & 0xFFu) * rows);
-        b.rowEnd = uni(min(b.rowEnd, b.row + rows));
+        b.rowEnd = uni(min(L.rows, b.row + rows));
     }
     // (a part past the item's last row: one batch, which run_bounds finds empty)
     return b;
