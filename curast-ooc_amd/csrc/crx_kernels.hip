@@ -2337,14 +2337,19 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(PU16 || V
     });
 }
 
-// Boxes of a mesh's units, computed once when the mesh is made: one wave per
-// unit, two triangles per lane and row, on the positions the raster stages
-// decode.
+// Boxes of a mesh's units, computed once when the mesh is made or a server's
+// node uploaded, on the positions the raster stages decode: one workgroup per
+// unit, a wave per row, two triangles per lane whose loads overlap.  A node of
+// 180,000 triangles has 176 units, so its kernel is as long as the dependent
+// loads of one wave: with a wave per unit, row after row, 20 us, which every
+// streamed node's first draw waited for.
 template <bool PU16>
-__global__ __launch_bounds__(256) void k_unit_bounds(DrawItem it, uint32_t numUnits, UnitBox* __restrict__ out) {
-    const uint32_t u = uni(blockIdx.x * 4u + threadIdx.x / kWave);
-    if (u >= numUnits) return;
+__global__ __launch_bounds__(kUnitRows * kWave) void k_unit_bounds(DrawItem it, UnitBox* __restrict__ out) {
+    __shared__ int32_t keys[6];                // the unit's lower and upper corner
+    const uint32_t u = blockIdx.x;
     const uint32_t lane = threadIdx.x & (kWave - 1);
+    if (threadIdx.x < 6) keys[threadIdx.x] = threadIdx.x < 3 ? 0x7FFFFFFF : (int32_t)0x80000000;
+    __syncthreads();
     RunLayout L;
     L.rowTris = it.rowTris;
     L.unitRows = it.unitRows;
@@ -2354,41 +2359,52 @@ __global__ __launch_bounds__(256) void k_unit_bounds(DrawItem it, uint32_t numUn
     L.firstUnit = 0u;
     S1Item si{};
     si.numTriangles = it.numTriangles;
-    int32_t lo[3] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF};
-    int32_t hi[3] = {(int32_t)0x80000000, (int32_t)0x80000000, (int32_t)0x80000000};
     RunBatch b = run_first(L, u);
-    for (; b.row < b.rowEnd; b.row++) {
-        uint32_t base, end;
-        run_bounds(si, L, b, base, end);
-        for (uint32_t t = base + lane; t < end; t += kWave) {
-            uint32_t v[3];
+    b.row = uni(b.row + threadIdx.x / kWave);
+    uint32_t base = 0u, end = 0u;
+    if (b.row < b.rowEnd) run_bounds(si, L, b, base, end);
+    if (base < end) {
+        int32_t lo[3] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF};
+        int32_t hi[3] = {(int32_t)0x80000000, (int32_t)0x80000000, (int32_t)0x80000000};
+        uint32_t v[6];
+        #pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t t = min(base + lane + (uint32_t)h * kWave, end - 1u);
             if constexpr (PU16) {
                 const uint64_t off = (uint64_t)it.bitsPerIndex * (3ull * t);
                 #pragma unroll
                 for (int j = 0; j < 3; j++)
-                    v[j] = bit_read(it.indices, off + (uint64_t)j * it.bitsPerIndex, it.bitsPerIndex) + it.indexMin;
+                    v[3 * h + j] =
+                        bit_read(it.indices, off + (uint64_t)j * it.bitsPerIndex, it.bitsPerIndex) + it.indexMin;
             } else {
                 #pragma unroll
-                for (int j = 0; j < 3; j++) v[j] = it.indexMask ? it.indices[3ull * t + j] : 3u * t + (uint32_t)j;
+                for (int j = 0; j < 3; j++)
+                    v[3 * h + j] = it.indexMask ? it.indices[3ull * t + j] : 3u * t + (uint32_t)j;
             }
+        }
+        #pragma unroll
+        for (int j = 0; j < 6; j++) {
+            const f3 p = PU16 ? load_pos_pu16(it.positions, v[j], it.cf, it.amin) : load_pos_g(it.positions, v[j]);
+            const int32_t k[3] = {fkey(p.x), fkey(p.y), fkey(p.z)};
             #pragma unroll
-            for (int j = 0; j < 3; j++) {
-                const f3 p = PU16 ? load_pos_pu16(it.positions, v[j], it.cf, it.amin) : load_pos_g(it.positions, v[j]);
-                const int32_t k[3] = {fkey(p.x), fkey(p.y), fkey(p.z)};
-                #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    lo[c] = min(lo[c], k[c]);
-                    hi[c] = max(hi[c], k[c]);
-                }
+            for (int c = 0; c < 3; c++) {
+                lo[c] = min(lo[c], k[c]);
+                hi[c] = max(hi[c], k[c]);
+            }
+        }
+        #pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const int32_t l = wave_min_i(lo[c]), h = wave_max_i(hi[c]);
+            if (lane == 0) {
+                atomicMin(keys + c, l);
+                atomicMax(keys + 3 + c, h);
             }
         }
     }
-    #pragma unroll
-    for (int c = 0; c < 3; c++) {
-        lo[c] = wave_min_i(lo[c]);
-        hi[c] = wave_max_i(hi[c]);
-    }
-    if (lane != 0) return;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const int32_t* lo = keys;
+    const int32_t* hi = keys + 3;
     UnitBox r{};
     float M = 0.0f;
     bool finite = true;
@@ -3722,10 +3738,10 @@ hipError_t launch_cull_units(const RasterParams& P, hipStream_t stream) {
 }
 
 hipError_t launch_unit_bounds(const DrawItem& item, bool pu16, uint32_t numUnits, UnitBox* out, hipStream_t stream) {
-    const uint32_t blocks = (numUnits + 3u) / 4u;
     (void)hipGetLastError();   // an error that an earlier call left behind is not this launch's
-    if (pu16) hipLaunchKernelGGL(k_unit_bounds<true>, dim3(blocks), dim3(256), 0, stream, item, numUnits, out);
-    else hipLaunchKernelGGL(k_unit_bounds<false>, dim3(blocks), dim3(256), 0, stream, item, numUnits, out);
+    const dim3 grid(numUnits), block(kUnitRows * kWave);
+    if (pu16) hipLaunchKernelGGL(k_unit_bounds<true>, grid, block, 0, stream, item, out);
+    else hipLaunchKernelGGL(k_unit_bounds<false>, grid, block, 0, stream, item, out);
     return hipGetLastError();
 }
 

@@ -848,7 +848,8 @@ crx_status crx_server_start(crx_server* s) {
         hipError_t e = hipMalloc(&s->cache, (size_t)s->numSlots * slot);
         if (e != hipSuccess) { s->cache = nullptr; return fail(CRX_OUT_OF_MEMORY, std::string("node cache: ") + hipGetErrorString(e)); }
     }
-    for (size_t i = 0; i < s->nodes.size(); i++) {
+    // (a scene that no draw lists units of needs no boxes)
+    for (size_t i = 0; s->totalTriangles >= kListMinTris && i < s->nodes.size(); i++) {
         Node& n = s->nodes[i];
         // nodes cut from one grid have the same indices, in one buffer or in copies
         const Node* before = i ? &s->nodes[i - 1] : nullptr;
