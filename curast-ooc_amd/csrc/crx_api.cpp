@@ -329,6 +329,68 @@ uint64_t pair_layout(DrawItem& it, uint32_t rowHint, uint32_t stripRows, uint32_
     return (uint64_t)it.strips * it.unitSegs;
 }
 
+// Workgroups that share the instances of a batch in a draw of meshes drawn over
+// many instances (k_stage1).  In one share a wave takes all instances of its
+// mesh in turn, so a mesh of few, large triangles (in pixels) holds the draw up
+// long after the others are through.  As many shares are taken as bring the
+// longest wave's work down to the mean of the chip's resident waves, by a rough
+// cost per wave and instance: the filter, and for triangles that it leaves the
+// exact code and the samples of their boxes, from the size on the screen of
+// up to four instances of each mesh.  At most one share per four instances,
+// which then take no box tests, and at most 16 rounds of waves.
+// Frames in one share, as this rule has it, and in one share per four instances:
+// 30 instances of 500,000 triangles 81, 81 (1 share) and 150 us, 53 of 204,000
+// 69, 75 (2) and 129, 1000 of 20,000 536, 148 (23) and 212, 600 nodes of 24
+// meshes 666, 396 (4) and 400, 912 nodes of 14 meshes 1049, 460 (6) and 408 in
+// ten; 3000 instances of a 1 M-triangle mesh 1087 in one, 1280 in two.
+uint32_t instance_shares(const crx_context* ctx, const DrawPlan& D, const crx_cmesh* list, int instanced,
+                         const crx_mat4* transforms, const crx_render_target& target) {
+    const double focal = 0.5 * std::fabs((double)target.proj.m[5]) * target.height;
+    const double screen = (double)target.width * target.height;
+    double total = 0.0, longest = 0.0, tris = 0.0;
+    for (uint32_t k = 0; k < D.numItems; k++) {
+        const crx_cmesh& m = list[k];
+        const uint32_t count = instanced ? (uint32_t)m.instances.count : 1u;
+        if (count == 0 || m.numTriangles == 0) continue;
+        const double lo[3] = {m.aabb.min.x, m.aabb.min.y, m.aabb.min.z}, hi[3] = {m.aabb.max.x, m.aabb.max.y, m.aabb.max.z};
+        double c[3], r2 = 0.0;
+        for (int a = 0; a < 3; a++) {
+            c[a] = 0.5 * (lo[a] + hi[a]);
+            r2 += 0.25 * (hi[a] - lo[a]) * (hi[a] - lo[a]);
+        }
+        const uint32_t samples = std::min(count, 4u);
+        double mean = 0.0;
+        for (uint32_t s = 0; s < samples; s++) {
+            const uint32_t j = samples > 1 ? (uint32_t)((uint64_t)s * (count - 1u) / (samples - 1u)) : 0u;
+            const float* x = transforms[(uint32_t)m.instances.offset + j].m;
+            double scale2 = 0.0;
+            for (int a = 0; a < 3; a++)
+                scale2 = std::max(scale2, (double)x[4 * a] * x[4 * a] + (double)x[4 * a + 1] * x[4 * a + 1] +
+                                              (double)x[4 * a + 2] * x[4 * a + 2]);
+            const double depth = -(x[2] * c[0] + x[6] * c[1] + x[10] * c[2] + x[14]);
+            const double radius2 = r2 * scale2;
+            // pixels of the box's sphere, and of a triangle facing the view (half of them)
+            double area = 0.0;
+            if (radius2 > 0.0) area = depth * depth <= radius2 ? screen : 3.1416 * radius2 * focal * focal / (depth * depth);
+            if (depth * depth > radius2 && depth < 0.0) area = 0.0;            // behind the camera
+            if (!(area >= 0.0)) area = 0.0;                                    // no usable box
+            const double pixels = std::min(area, screen) / (0.5 * m.numTriangles);
+            const double box = 6.0 * pixels;                                   // samples of its box
+            mean += (110.0 + std::min(1.0, 4.0 * pixels) * (280.0 + (box > 128.0 ? 0.0 : 30.0 * box))) / samples;
+        }
+        const double waves = std::ceil(m.numTriangles / 64.0);
+        total += waves * count * mean;
+        longest = std::max(longest, count * mean);
+        tris += m.numTriangles;
+    }
+    if (total <= 0.0) return 1u;
+    const double waves = std::max<double>(1.0, (double)D.g1 * (D.block / 64));
+    const double resident = ctx->numCUs * 28.0;
+    const double fine = std::ceil(std::ceil(D.tris / tris) / 4.0);     // (the mean number of instances of a triangle)
+    const double want = std::min({std::floor(longest * resident / total + 0.5), fine, 16.0 * resident / waves, 1024.0});
+    return (uint32_t)std::max(1.0, want);
+}
+
 // Host records and metadata layout of a draw of numViews >= 1 views sharing
 // one instance list (transforms view-major).  No device work.
 crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMeshes, const crx_cmesh* instances,
@@ -509,26 +571,8 @@ crx_status plan_draw(crx_context* ctx, const crx_cmesh* meshes, uint32_t numMesh
         D.g1 = grid_for(ctx, sched.wavesPerCU, D.block / 64);
         if (D.g1 > D.batches) D.g1 = (uint32_t)D.batches;
     }
-    if (D.instanceBoxes && numViews == 1) {
-        // A batch's instances are shared by several workgroups.  Shares of
-        // about four instances take no box tests and spread the large
-        // triangles of near instances over the chip (600 nodes of 24 meshes:
-        // 720 us per frame in one share, 406 in four, 393 in six, 409 in
-        // eight, where the vertices are fetched too often).  A draw of so many
-        // instances that such shares are past number keeps long ones, which the box
-        // tests thin out, as few as give the chip two rounds of waves (3000
-        // instances of a 1 M-triangle mesh: 1247 us per frame in one share,
-        // 1280 in two, 1474 in eight).
-        uint64_t tris = 0;
-        for (uint32_t k = 0; k < D.numItems; k++) tris += list[k].numTriangles;
-        const uint64_t waves = std::max<uint64_t>(1, (uint64_t)D.g1 * (D.block / 64));
-        const uint64_t resident = (uint64_t)ctx->numCUs * 28u;
-        const uint64_t mean = tris ? (D.tris + tris - 1) / tris : 1;      // instances of a triangle
-        const uint64_t fine = std::min<uint64_t>((mean + 3) / 4, 1024);
-        D.instanceShares = (uint32_t)(waves * fine <= 16 * resident
-                                          ? fine
-                                          : std::min<uint64_t>(fine, std::max<uint64_t>(1, 2 * resident / waves)));
-    }
+    if (D.instanceBoxes && numViews == 1)
+        D.instanceShares = instance_shares(ctx, D, list, instanced, transforms, targets[0]);
     D.g1 = (D.g1 + 7u) & ~7u;   // the stage-1 XCD split assumes a multiple of 8 workgroups
     D.g2 = grid_for(ctx, tu.stage2_waves_per_cu, 4);
     D.g3 = grid_for(ctx, tu.stage3_waves_per_cu, 4);

@@ -152,6 +152,33 @@ def test_many_instances(ctx, large):
     sphere.close()
 
 
+@pytest.mark.parametrize("rings,segments,count", [(500, 500, 30), (163, 625, 53), (100, 100, 40), (64, 64, 120)])
+def test_shares_of_one_mesh(ctx, rings, segments, count):
+    """One mesh: as many shares as its waves leave of the 28 per CU that the chip
+    holds (none for a mesh that fills it), at most one per four instances."""
+    mesh = crx.Mesh(ctx, *wl.sphere_mesh(rings, segments))
+    worlds = wl.instance_transforms(count, extent=200.0)
+    pose = ((350.0, 350.0, 350.0), (100.0, 100.0, 100.0))
+    got = _draw(ctx, [(mesh, w) for w in worlds], [(800, 600)], pose)
+    waves = -(-mesh.num_triangles // 64)
+    want = max(1, min(int(28 * ctx.num_cus / waves + 0.5), -(-count // 4)))
+    mesh.close()
+    assert (got.route, got.shares) == (crx.STAGE1_PLAIN, want)
+
+
+def test_shares_of_small_meshes_beside_a_large_one(ctx):
+    """A mesh of few triangles of many pixels takes all its instances in a handful of
+    waves, long after the large mesh is through: the draw is shared."""
+    large, small = crx.Mesh(ctx, *wl.sphere_mesh(320, 320)), crx.Mesh(ctx, *wl.sphere_mesh(20, 20))
+    worlds = list(wl.instance_transforms(64, extent=30.0))
+    pose = ((15.0, 18.0, -12.0), (15.0, 12.0, 15.0))
+    alone = _draw(ctx, [(large, w) for w in worlds[:32]], [(1365, 769)], pose)
+    both = _draw(ctx, [(large, w) for w in worlds[:32]] + [(small, w) for w in worlds[32:]], [(1365, 769)], pose)
+    large.close()
+    small.close()
+    assert alone.shares == max(1, min(8, int(28 * ctx.num_cus / 3200 + 0.5))) and both.shares > alone.shares
+
+
 def test_nothing_to_draw(ctx):
     scene = crx.Scene(ctx)
     fb = ctx.alloc(8 * 64)
