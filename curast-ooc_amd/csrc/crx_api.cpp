@@ -336,18 +336,22 @@ uint64_t pair_layout(DrawItem& it, uint32_t rowHint, uint32_t stripRows, uint32_
 // longest wave's work down to the mean of the chip's resident waves, by a rough
 // cost per wave and instance: the filter, and for triangles that it leaves the
 // exact code and the samples of their boxes, from the size on the screen of
-// up to four instances of each mesh.  At most one share per four instances,
-// which then take no box tests, and at most 16 rounds of waves.
+// up to four instances of each mesh.  Where the meshes' waves differ, so do a
+// mesh's instances, the nearest far above the mean that the samples give: up to
+// five times as many.  At most one share per four instances, which then take
+// no box tests, and at most 16 rounds of waves.
 // Frames in one share, as this rule has it, and in one share per four instances:
 // 30 instances of 500,000 triangles 81, 81 (1 share) and 150 us, 53 of 204,000
-// 69, 75 (2) and 129, 1000 of 20,000 536, 148 (23) and 212, 600 nodes of 24
-// meshes 666, 396 (4) and 400, 912 nodes of 14 meshes 1049, 460 (6) and 408 in
-// ten; 3000 instances of a 1 M-triangle mesh 1087 in one, 1280 in two.
+// 74, 83 (2) and 121, 1000 of 20,000 532, 146 (23) and 212, 600 nodes of 24
+// meshes 662, 393 (7) and 393 (408 in the 4 without the factor), these at
+// 3840x2160 1207, 970 (7) and 970, 912 nodes of 14 meshes 1046, 416 (14) and 413
+// (462 in the 6 without), 1500 nodes of 40 meshes 1192, 812 (7) and 857; 3000
+// instances of a 1 M-triangle mesh 1087 in one, 1280 in two.
 uint32_t instance_shares(const crx_context* ctx, const DrawPlan& D, const crx_cmesh* list, int instanced,
                          const crx_mat4* transforms, const crx_render_target& target) {
     const double focal = 0.5 * std::fabs((double)target.proj.m[5]) * target.height;
     const double screen = (double)target.width * target.height;
-    double total = 0.0, longest = 0.0, tris = 0.0;
+    double total = 0.0, longest = 0.0, tris = 0.0, all = 0.0;
     for (uint32_t k = 0; k < D.numItems; k++) {
         const crx_cmesh& m = list[k];
         const uint32_t count = instanced ? (uint32_t)m.instances.count : 1u;
@@ -382,12 +386,15 @@ uint32_t instance_shares(const crx_context* ctx, const DrawPlan& D, const crx_cm
         total += waves * count * mean;
         longest = std::max(longest, count * mean);
         tris += m.numTriangles;
+        all += waves;
     }
     if (total <= 0.0) return 1u;
     const double waves = std::max<double>(1.0, (double)D.g1 * (D.block / 64));
     const double resident = ctx->numCUs * 28.0;
     const double fine = std::ceil(std::ceil(D.tris / tris) / 4.0);     // (the mean number of instances of a triangle)
-    const double want = std::min({std::floor(longest * resident / total + 0.5), fine, 16.0 * resident / waves, 1024.0});
+    const double spread = longest * all / total;                       // 1 for one mesh, 2.4 and more for the nodes above
+    const double even = longest * resident / total * std::min(5.0, spread * spread);
+    const double want = std::min({std::floor(even + 0.5), fine, 16.0 * resident / waves, 1024.0});
     return (uint32_t)std::max(1.0, want);
 }
 
