@@ -2212,7 +2212,7 @@ struct LeftTris {
 // kept with them: gathered again from memory they made the kernel fetch 600
 // MB in place of 520 and wait (143 us against 134).
 // Stage 1 of that terrain 195 -> 139 us (VALU instructions 112 M -> 54 M, 3.7
-// TB/s fetched), of the 400 M-triangle one's 1.5% in view 79 -> 66.
+// TB/s fetched), of the 400 M-triangle one's 1.8% in view 79 -> 66.
 //
 // Several views: a unit is drawn once for every view that may see it, where
 // k_stage1_views tests every 64 triangles against every view.  Their triangles
@@ -2425,13 +2425,14 @@ constexpr uint32_t kCullChunk = 1024;    // units per workgroup, one per lane
 
 // Lists the units of a draw that a view may see (workgroup c * views + v:
 // view v, chunk c; the views of a chunk follow each other, so that those that
-// draw a unit find it in the caches; view_may_see: a unit is dropped only when every triangle in it is culled by its own exact
-// tests), and marks those wholly inside it (kUnitInside; every instance's,
-// where the item has several).  One append per workgroup of 1024 units: the
-// returning atomics on the one counter take 6 ns each.  A terrain flown over
-// has most of its units outside the view; their geometry is not read.
-// Stage 1 of the 400 M-triangle terrain at 1080p, which sees 1.5% of its
-// units: 1457 us over all units, 81 over the listed ones plus 6 here.
+// draw a unit find it in the caches; view_may_see: a unit is dropped only when
+// every triangle in it is culled by its own exact tests), and marks those
+// wholly inside it (kUnitInside; every instance's, where the item has
+// several).  One append per workgroup of 1024 units: the returning atomics on
+// the one counter take 6 ns each.  A terrain flown over has most of its units
+// outside the view; their geometry is not read.  Stage 1 of the 400 M-triangle
+// terrain at 1080p, which sees 1.8% of its units: 1457 us over all units, 65
+// over the listed ones plus 7 here.
 __global__ __launch_bounds__(1024) void k_cull_units(RasterParams P) {
     __shared__ uint32_t counts[kCullChunk / kWave];
     __shared__ uint32_t listBase;
